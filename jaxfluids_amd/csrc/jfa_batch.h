@@ -55,18 +55,6 @@ struct BatchArgs {
     const unsigned long long* wave_max;  // per case, 3 slots: WAVESPEED maxima of W_in (nullable)
 };
 
-// Wave-uniform copies in scalar registers.  The records are read with vector loads (the
-// kernel's stores could alias them as far as the compiler knows); readfirstlane moves each
-// field into an SGPR, so the per-case constants do not occupy vector registers.
-__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ int64_t uni(int64_t v) {
-    const uint64_t u = (uint64_t)v;
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
-    return (int64_t)(((uint64_t)hi << 32) | lo);
-}
-__device__ __forceinline__ double uni(double v) { return __longlong_as_double(uni((int64_t)__double_as_longlong(v))); }
-
 __device__ __forceinline__ Case2D load_case(const Case2D* __restrict__ p) {
     const Case2D r = *p;
     Case2D c;
@@ -120,23 +108,6 @@ __device__ __forceinline__ Geo geo_of(const Case2D& cs) {
     G.active[1] = 1;
     G.active[2] = 0;
     return G;
-}
-
-// Loads and stores at a wave-uniform base pointer plus a per-lane byte offset.  The base
-// lives in scalar registers (it carries the plane, field and stencil-tap offsets), the
-// lane part is one 32-bit vector register (the column), so every access of a face window
-// compiles to the scalar-base form and the march keeps no per-tap vector addresses.
-template <class T>
-__device__ __forceinline__ double ldo(const T* __restrict__ base, uint32_t voff) {
-    const T* p = reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + voff);
-    JFA_ACCESS(p, sizeof(T));
-    return static_cast<double>(*p);
-}
-template <class T>
-__device__ __forceinline__ void sto(T* __restrict__ base, uint32_t voff, double v) {
-    T* p = reinterpret_cast<T*>(reinterpret_cast<char*>(base) + voff);
-    JFA_ACCESS(p, sizeof(T));
-    *p = static_cast<T>(v);
 }
 
 // Flux of one face along AXIS (stride st): window cells -3..2 relative to the cell right of

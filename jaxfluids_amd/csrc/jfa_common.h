@@ -67,14 +67,39 @@ static inline int check_launch() {
 
 // Hooks for a host build of these sources (the test suite's CPU emulation of the kernels):
 // JFA_ACCESS(p, bytes) sees every state load and store, JFA_OPAQUE(x) hides a value from the
-// optimiser, JFA_WAVES_PER_EU(n) asks the compiler to fit n waves per SIMD.  In the library
-// JFA_ACCESS is empty, JFA_OPAQUE is an empty asm statement that keeps per-tap address
-// arithmetic from being hoisted out of march loops, and JFA_WAVES_PER_EU the amdgpu attribute.
+// optimiser (JFA_OPAQUE_S a wave-uniform one, in scalar registers), JFA_WAVES_PER_EU(n) asks the
+// compiler to fit n waves per SIMD.  In the library JFA_ACCESS is empty, JFA_OPAQUE is an empty asm
+// statement that keeps per-tap address arithmetic from being hoisted out of march loops, and
+// JFA_WAVES_PER_EU the amdgpu attribute.
 #ifndef JFA_ACCESS
 #define JFA_ACCESS(p, bytes)
 #endif
 #ifndef JFA_OPAQUE
 #define JFA_OPAQUE(x) asm volatile("" : "+v"(x))
+#endif
+#ifndef JFA_OPAQUE_S
+#ifdef __HIP__
+#define JFA_OPAQUE_S(x) asm volatile("" : "+s"(x))
+#else
+#define JFA_OPAQUE_S(x) ((void)0)
+#endif
+#endif
+// JFA_SCHED_BARRIER() keeps the instruction scheduler from moving code across it; JFA_WAVE_FENCE()
+// orders the wavefront's LDS accesses across lanes (the hardware runs them in order, so the library
+// only stops the compiler; a host build lets the wave's lanes meet).
+#ifndef JFA_SCHED_BARRIER
+#ifdef __HIP__
+#define JFA_SCHED_BARRIER() __builtin_amdgcn_sched_barrier(0)
+#else
+#define JFA_SCHED_BARRIER() ((void)0)
+#endif
+#endif
+#ifndef JFA_WAVE_FENCE
+#ifdef __HIP__
+#define JFA_WAVE_FENCE() __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront")
+#else
+#define JFA_WAVE_FENCE() ((void)__builtin_amdgcn_readfirstlane(0))
+#endif
 #endif
 #ifndef JFA_WAVES_PER_EU
 #define JFA_WAVES_PER_EU(n) __attribute__((amdgpu_waves_per_eu(n)))
@@ -84,6 +109,34 @@ template <class T>
 __device__ __forceinline__ double ld(const T* __restrict__ p, int64_t i) {
     JFA_ACCESS(p + i, sizeof(T));
     return static_cast<double>(p[i]);
+}
+
+// Wave-uniform copies in scalar registers: readfirstlane moves a value that is the same in every
+// lane of the wave, but that the compiler cannot know to be, out of the vector registers.
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ int64_t uni(int64_t v) {
+    const uint64_t u = (uint64_t)v;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
+    return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ double uni(double v) { return __longlong_as_double(uni((int64_t)__double_as_longlong(v))); }
+
+// Loads and stores at a wave-uniform base pointer plus a per-lane byte offset.  The base
+// lives in scalar registers (it carries the plane, field and stencil-tap offsets), the
+// lane part is one 32-bit vector register (the column), so every access of a face window
+// compiles to the scalar-base form and the march keeps no per-tap vector addresses.
+template <class T>
+__device__ __forceinline__ double ldo(const T* __restrict__ base, uint32_t voff) {
+    const T* p = reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + voff);
+    JFA_ACCESS(p, sizeof(T));
+    return static_cast<double>(*p);
+}
+template <class T>
+__device__ __forceinline__ void sto(T* __restrict__ base, uint32_t voff, double v) {
+    T* p = reinterpret_cast<T*>(reinterpret_cast<char*>(base) + voff);
+    JFA_ACCESS(p, sizeof(T));
+    *p = static_cast<T>(v);
 }
 
 // Face extents along axis a: N_a+1 on a, interior extents elsewhere.

@@ -124,13 +124,17 @@ __device__ __forceinline__ double fsqrt(double x) {
 //   into g_k = d_k delta_k.
 constexpr double kQ = 13.0 / 3.0;
 
-// c + sum_k omega_k delta_k from the scaled indicators b0..b2 and g0..g2.  With q_k = b_k + eps
-// (WENO-Z) the weights are omega_k ~ d_k (1 + tau5/q_k) ~ d_k e_k, e_k = P + tau5 prod_{j != k} q_j
-// and P = q0 q1 q2; with q_k = b_k^2 + eps (WENO-JS) omega_k ~ d_k / q_k ~ d_k prod_{j != k} q_j.
+// Unnormalised weights e_k (omega_k ~ d_k e_k) from the slopes S_k and the scaled squares
+// Q_k = (13/3) D_k^2 of a stencil's three sub-stencils, 4 beta_k = S_k^2 + Q_k.
+//   WENO-Z:  q_k = 4 beta_k + eps (Q_k comes with eps added, sq()), omega_k ~ d_k (1 + tau5/q_k) ~ d_k e_k,
+//            e_k = P + tau5 prod_{j != k} q_j, P = q0 q1 q2, tau5 = |q0 - q2|;
+//   WENO-JS: q_k = (4 beta_k)^2 + eps, omega_k ~ d_k / q_k ~ d_k prod_{j != k} q_j.
+// The mirrored stencil (the other side of the same cell) has the same weights with e0 and e2
+// exchanged, so a cell's two states share them (weno5_cell).
 template <int STENCIL>
-__device__ __forceinline__ double weno5_combine(double b0, double b1, double b2, double g0, double g1, double g2,
-                                                double c, const double eps_z, const double eps_js) {
-    double e0, e1, e2;
+__device__ __forceinline__ void weno5_weights(double S0, double S1, double S2, double Q0, double Q1, double Q2,
+                                              const double eps_js, double& e0, double& e1, double& e2) {
+    const double b0 = fma(S0, S0, Q0), b1 = fma(S1, S1, Q1), b2 = fma(S2, S2, Q2);
     if constexpr (STENCIL == JFA_WENO5_JS) {
         const double q0 = fma(b0, b0, eps_js), q1 = fma(b1, b1, eps_js), q2 = fma(b2, b2, eps_js);
         e0 = q1 * q2;
@@ -138,15 +142,31 @@ __device__ __forceinline__ double weno5_combine(double b0, double b1, double b2,
         e2 = q0 * q1;
     } else {
         const double tau5 = fabs(b0 - b2);
-        const double q0 = b0 + eps_z, q1 = b1 + eps_z, q2 = b2 + eps_z;
-        const double p12 = q1 * q2, p02 = q0 * q2, p01 = q0 * q1;
-        const double P = p01 * q2;
+        const double p12 = b1 * b2, p02 = b0 * b2, p01 = b0 * b1;
+        const double P = p01 * b2;
         e0 = fma(tau5, p12, P);
         e1 = fma(tau5, p02, P);
         e2 = fma(tau5, p01, P);
     }
+}
+
+// (13/3) D^2, with WENO-Z's epsilon added (it joins the indicator for free in the fma)
+template <int STENCIL>
+__device__ __forceinline__ double weno5_sq(double D, const double eps_z) {
+    return STENCIL == JFA_WENO5_Z ? fma(kQ * D, D, eps_z) : (kQ * D) * D;
+}
+
+// c + sum_k omega_k delta_k of the stencil around c whose first differences are d0..d3, outermost
+// downwind last: the linear weights are folded into g_k = 10 d_k delta_k, and the weights' sum is
+// e0 + 6 e1 + 3 e2.
+__device__ __forceinline__ double weno5_state(double e0, double e1, double e2, double d0, double d1, double d2,
+                                              double d3, double c) {
+    const double t = d2 + d2;
+    const double g0 = fma(5.0 / 6.0, d1, (-1.0 / 3.0) * d0);
+    const double g1 = d1 + t;
+    const double g2 = fma(-0.5, d3, t);
     const double num = fma(e2, g2, fma(e1, g1, e0 * g0));
-    const double den = fma(0.3, e2, fma(0.6, e1, 0.1 * e0));
+    const double den = fma(3.0, e2, fma(6.0, e1, e0));
     return fma(num, rcp1(den), c);
 }
 
@@ -156,12 +176,10 @@ __device__ __forceinline__ double weno5(double a, double b, double c, double d, 
                                         const double eps_js) {
     const double d0 = b - a, d1 = c - b, d2 = d - c, d3 = e - d;
     const double D0 = d1 - d0, D1 = d2 - d1, D2 = d3 - d2;
-    const double S0 = fma(3.0, d1, -d0), S1 = d1 + d2, S2 = fma(-3.0, d2, d3);
-    const double b0 = fma(S0, S0, (kQ * D0) * D0), b1 = fma(S1, S1, (kQ * D1) * D1), b2 = fma(S2, S2, (kQ * D2) * D2);
-    const double g0 = fma(1.0 / 12.0, d1, (-1.0 / 30.0) * d0);
-    const double g1 = fma(0.2, d2, 0.1 * d1);
-    const double g2 = fma(0.2, d2, -0.05 * d3);
-    return weno5_combine<STENCIL>(b0, b1, b2, g0, g1, g2, c, eps_z, eps_js);
+    double e0, e1, e2;
+    weno5_weights<STENCIL>(fma(3.0, d1, -d0), d1 + d2, fma(-3.0, d2, d3), weno5_sq<STENCIL>(D0, eps_z),
+                           weno5_sq<STENCIL>(D1, eps_z), weno5_sq<STENCIL>(D2, eps_z), eps_js, e0, e1, e2);
+    return weno5_state(e0, e1, e2, d0, d1, d2, d3, c);
 }
 
 // Left (j = 0: cells -3..1) and right (j = 1: cells 2..-2) states of one face from its
@@ -172,24 +190,30 @@ template <int STENCIL>
 __device__ __forceinline__ void weno5_pair(const double v[6], const double eps_z, const double eps_js, double& L,
                                            double& R) {
     const double d0 = v[1] - v[0], d1 = v[2] - v[1], d2 = v[3] - v[2], d3 = v[4] - v[3], d4 = v[5] - v[4];
-    const double E0 = d1 - d0, E1 = d2 - d1, E2 = d3 - d2, E3 = d4 - d3;
-    const double Q1 = (kQ * E1) * E1, Q2 = (kQ * E2) * E2;
-    {  // left: stencil v0..v4, centre v2
-        const double S0 = fma(3.0, d1, -d0), S1 = d1 + d2, S2 = fma(-3.0, d2, d3);
-        const double b0 = fma(S0, S0, (kQ * E0) * E0), b1 = fma(S1, S1, Q1), b2 = fma(S2, S2, Q2);
-        const double g0 = fma(1.0 / 12.0, d1, (-1.0 / 30.0) * d0);
-        const double g1 = fma(0.2, d2, 0.1 * d1);
-        const double g2 = fma(0.2, d2, -0.05 * d3);
-        L = weno5_combine<STENCIL>(b0, b1, b2, g0, g1, g2, v[2], eps_z, eps_js);
-    }
-    {  // right: stencil v5..v1, centre v3; its differences are (-d4, -d3, -d2, -d1)
-        const double S0 = fma(-3.0, d3, d4), S1 = d3 + d2, S2 = fma(3.0, d2, -d1);
-        const double b0 = fma(S0, S0, (kQ * E3) * E3), b1 = fma(S1, S1, Q2), b2 = fma(S2, S2, Q1);
-        const double g0 = fma(-1.0 / 12.0, d3, (1.0 / 30.0) * d4);
-        const double g1 = fma(-0.2, d2, -0.1 * d3);
-        const double g2 = fma(-0.2, d2, 0.05 * d1);
-        R = weno5_combine<STENCIL>(b0, b1, b2, g0, g1, g2, v[3], eps_z, eps_js);
-    }
+    const double Q0 = weno5_sq<STENCIL>(d1 - d0, eps_z), Q1 = weno5_sq<STENCIL>(d2 - d1, eps_z);
+    const double Q2 = weno5_sq<STENCIL>(d3 - d2, eps_z), Q3 = weno5_sq<STENCIL>(d4 - d3, eps_z);
+    double e0, e1, e2;
+    // left: stencil v0..v4, centre v2
+    weno5_weights<STENCIL>(fma(3.0, d1, -d0), d1 + d2, fma(-3.0, d2, d3), Q0, Q1, Q2, eps_js, e0, e1, e2);
+    L = weno5_state(e0, e1, e2, d0, d1, d2, d3, v[2]);
+    // right: stencil v5..v1, centre v3; its differences are (-d4, -d3, -d2, -d1)
+    weno5_weights<STENCIL>(fma(-3.0, d3, d4), d3 + d2, fma(3.0, d2, -d1), Q3, Q2, Q1, eps_js, e0, e1, e2);
+    R = weno5_state(e0, e1, e2, -d4, -d3, -d2, -d1, v[3]);
+}
+
+// The two states a cell gives its faces, from its five cells (a .. e, centre c): lo is the right
+// state of the face below c, hi the left state of the face above.  Both stencils are a..e, one
+// mirrored, so the indicators and weights are evaluated once: 63 FP64 issue slots against 81 for
+// a face's pair (a reciprocal estimate counted as 4).
+template <int STENCIL>
+__device__ __forceinline__ void weno5_cell(double a, double b, double c, double d, double e, const double eps_z,
+                                           const double eps_js, double& lo, double& hi) {
+    const double d0 = b - a, d1 = c - b, d2 = d - c, d3 = e - d;
+    double e0, e1, e2;
+    weno5_weights<STENCIL>(fma(3.0, d1, -d0), d1 + d2, fma(-3.0, d2, d3), weno5_sq<STENCIL>(d1 - d0, eps_z),
+                           weno5_sq<STENCIL>(d2 - d1, eps_z), weno5_sq<STENCIL>(d3 - d2, eps_z), eps_js, e0, e1, e2);
+    hi = weno5_state(e0, e1, e2, d0, d1, d2, d3, c);
+    lo = weno5_state(e2, e1, e0, -d3, -d2, -d1, -d0, c);
 }
 
 // ---------------------------------------------------------------- further stencils
@@ -591,6 +615,7 @@ struct Frozen {
     double P[5];            // primes_ave
     double H, g, c, cc, q2; // enthalpy, grueneisen, c, c^2, velocity_square
     double inv_c, rcc;      // 1/c and c^2 * rho_ave
+    double m;               // 1/(rho_ave c)
 };
 
 __device__ __forceinline__ double total_enthalpy(const double W[5], const Params& prm) {
@@ -612,6 +637,7 @@ __device__ __forceinline__ void frozen_state(const double WL[5], const double WR
         f.inv_c = f.P[0] * r;
         f.cc = f.c * f.c;       // :230
         f.rcc = gp;
+        f.m = r;
         if (FULL) {
             f.g = prm.gm1;                                             // :216-218
             f.H = total_enthalpy(f.P, prm);                            // :219-222
@@ -634,6 +660,7 @@ __device__ __forceinline__ void frozen_state(const double WL[5], const double WR
         f.inv_c = rsq1(f.cc);
         f.c = f.cc * f.inv_c;                                                      // :275
         f.rcc = f.cc * f.P[0];
+        f.m = f.inv_c * rcp1(f.P[0]);
         if (FULL) {
             f.H = (sL * total_enthalpy(WL, prm) + sR * total_enthalpy(WR, prm)) * rho_div;  // :250
             f.q2 = f.P[1] * f.P[1] + f.P[2] * f.P[2] + f.P[3] * f.P[3];                    // :271
@@ -727,14 +754,15 @@ __device__ __forceinline__ void signal_speeds(int kind, double uL, double uR, do
             SL = uL - aL * qL;
             SR = uR + aR * qR;
         } break;
-        default: {  // EINFELDT :125-132
-            const double yL = rsq1(rL), yR = rsq1(rR);
-            const double sL = rL * yL, sR = rR * yR;  // sqrt(rho)
-            const double one_dens = rcp1(sL + sR);
-            const double eta2 = 0.5 * sL * sR * one_dens * one_dens;
-            const double u_bar = (sL * uL + sR * uR) * one_dens;
+        default: {  // EINFELDT :125-132, with the sqrt(rho) averages as weights of the ratio
+            // s = sqrt(rho_R / rho_L): w_L = 1/(1 + s), w_R = s w_L (one inverse square root less;
+            // NaN as sqrt(rho) is if either density is negative)
+            const double s = rR * rsq1(fmin(rL, rR) * fabs(fmax(rL, rR)));
+            const double wL = rcp1(1.0 + s);
+            const double wR = s * wL;
+            const double u_bar = fma(wL, uL, wR * uR);
             const double du = uR - uL;
-            const double d_bar = fsqrt((sL * aL * aL + sR * aR * aR) * one_dens + eta2 * (du * du));
+            const double d_bar = fsqrt(fma(wL, aL * aL, fma(wR, aR * aR, (0.5 * wL * wR) * (du * du))));
             SL = fmin(u_bar - d_bar, uL - aL);
             SR = fmax(u_bar + d_bar, uR + aR);
         } break;
@@ -761,7 +789,8 @@ __device__ __forceinline__ void signal_speeds_davis2(double uL, double uR, doubl
 // With d = SK - u and inv = 1/(SK - Ss):
 //   pre = rho d inv                                  (:52)
 //   U*_4 = pre (E/rho + (Ss - u)(Ss + p/(rho d)))   (:59)  = inv (d E + (Ss - u)(rho d Ss + p))
-template <int AXIS>
+// UW: U = cons(W), so q = rho u is the normal momentum and U, U* share the tangential velocities.
+template <int AXIS, bool UW = false>
 __device__ __forceinline__ void hllc_star_flux(const double W[5], const double U[5], double SK, double S_clip,
                                                double Ss, double F[5]) {
     constexpr int v = Ax<AXIS>::v, m0 = Ax<AXIS>::m0, m1 = Ax<AXIS>::m1;
@@ -770,21 +799,36 @@ __device__ __forceinline__ void hllc_star_flux(const double W[5], const double U
     const double inv = rcp1(SK - Ss);
     const double rd = W[0] * d;
     const double pre = rd * inv;
-    double us[5];
-    us[0] = pre;
-    us[v] = pre * Ss;                                                   // :61
-    us[m0] = pre * W[m0];                                               // :62
-    us[m1] = pre * W[m1];                                               // :63
-    us[4] = inv * (d * U[4] + (Ss - uK) * (rd * Ss + W[4]));
-    physical_flux<AXIS>(W, U, F);                                       // :66
+    const double us4 = inv * fma(d, U[4], (Ss - uK) * fma(rd, Ss, W[4]));
+    if constexpr (UW) {
+        // F = phys(W, U) + S_clip (U* - U) (:66,76); the tangential momentum fluxes are the mass flux
+        // times the velocities
+        const double q = W[0] * uK;
+        F[0] = fma(S_clip, pre - W[0], q);
+        F[v] = fma(S_clip, fma(pre, Ss, -q), fma(q, uK, W[4]));
+        F[m0] = W[m0] * F[0];
+        F[m1] = W[m1] * F[0];
+        F[4] = fma(S_clip, us4 - U[4], uK * (U[4] + W[4]));
+    } else {
+        double us[5];
+        us[0] = pre;
+        us[v] = pre * Ss;      // :61
+        us[m0] = pre * W[m0];  // :62
+        us[m1] = pre * W[m1];  // :63
+        us[4] = us4;
+        physical_flux<AXIS>(W, U, F);  // :66
 #pragma unroll
-    for (int i = 0; i < 5; ++i) F[i] = F[i] + S_clip * (us[i] - U[i]);  // :76
+        for (int i = 0; i < 5; ++i) F[i] = F[i] + S_clip * (us[i] - U[i]);  // :76
+    }
 }
 
 // HLLC._solve_riemann_problem_xi_single_phase (HLLC.py:80-126).  The blend
 // 0.5(1+sgn S*) F*_L + 0.5(1-sgn S*) F*_R equals F*_L for S*>0 and F*_R for S*<0 exactly,
-// so only the needed side is evaluated; S* == 0 averages both (:123-124).
-template <int AXIS>
+// so only the needed side is evaluated; S* == 0 averages both (:123-124).  The sides are a branch,
+// not a selection of the operands: neighbouring faces mostly agree on the side, and runs of
+// v_cndmask on VCC issue at 22 cycles each (4 when other instructions lie between, measured).
+// UW: U = cons(W), formed here for the side that needs it (UL, UR are not read).
+template <int AXIS, bool UW = false>
 __device__ __forceinline__ void hllc(const double WL[5], const double WR[5], const double UL[5],
                                      const double UR[5], const Params& prm, double F[5]) {
     constexpr int v = Ax<AXIS>::v;
@@ -796,19 +840,19 @@ __device__ __forceinline__ void hllc(const double WL[5], const double WR[5], con
     const double rdL = WL[0] * (SL - WL[v]);
     const double rdR = WR[0] * (SR - WR[v]);
     const double Ss = fdiv((WR[4] - WL[4]) + (WL[v] * rdL - WR[v] * rdR), rdL - rdR);
-    const bool left = Ss >= 0.0;
-    double Wk[5], Uk[5];
-#pragma unroll
-    for (int i = 0; i < 5; ++i) {
-        Wk[i] = left ? WL[i] : WR[i];
-        Uk[i] = left ? UL[i] : UR[i];
+    if (Ss >= 0.0) {
+        double U[5];
+        if constexpr (UW) cons_from_prim(WL, prm, U);
+        hllc_star_flux<AXIS, UW>(WL, UW ? U : UL, SL, fmin(SL, 0.0), Ss, F);
+    } else {
+        double U[5];
+        if constexpr (UW) cons_from_prim(WR, prm, U);
+        hllc_star_flux<AXIS, UW>(WR, UW ? U : UR, SR, fmax(SR, 0.0), Ss, F);
     }
-    const double Sk = left ? SL : SR;
-    const double Sclip = left ? fmin(SL, 0.0) : fmax(SR, 0.0);
-    hllc_star_flux<AXIS>(Wk, Uk, Sk, Sclip, Ss, F);
     if (Ss == 0.0) {
-        double FR[5];
-        hllc_star_flux<AXIS>(WR, UR, SR, fmax(SR, 0.0), Ss, FR);
+        double U[5], FR[5];
+        if constexpr (UW) cons_from_prim(WR, prm, U);
+        hllc_star_flux<AXIS, UW>(WR, UW ? U : UR, SR, fmax(SR, 0.0), Ss, FR);
 #pragma unroll
         for (int i = 0; i < 5; ++i) F[i] = 0.5 * F[i] + 0.5 * FR[i];
     }
@@ -939,11 +983,11 @@ __device__ __forceinline__ void ausmp(const double WL[5], const double WR[5], co
 // face kernels, so the HLLC and Rusanov kernels keep their code.
 constexpr int kRiemannExt = 100;
 
-template <int AXIS, int RIEMANN>
+template <int AXIS, int RIEMANN, bool UW = false>
 __device__ __forceinline__ void riemann(const double WL[5], const double WR[5], const double UL[5],
                                         const double UR[5], const Params& prm, double F[5]) {
     if constexpr (RIEMANN == JFA_HLLC) {
-        hllc<AXIS>(WL, WR, UL, UR, prm, F);
+        hllc<AXIS, UW>(WL, WR, UL, UR, prm, F);
     } else if constexpr (RIEMANN == kRiemannExt) {
         if (prm.riemann == JFA_HLL) hll<AXIS>(WL, WR, UL, UR, prm, F);
         else if (prm.riemann == JFA_HLLC_LM) hllc_lm<AXIS>(WL, WR, UL, UR, prm, F);
@@ -1100,13 +1144,77 @@ __device__ __forceinline__ int limit_face_state(double Wf[5], const double q1[5]
     return n;
 }
 
+// Schemes whose neighbouring faces share reconstructions (face_states' CARRY).
+template <int VAR, int STENCIL>
+constexpr bool kCarry = (STENCIL == JFA_WENO5_JS || STENCIL == JFA_WENO5_Z) &&
+                        (VAR == JFA_PRIMITIVE || VAR == JFA_CHAR_PRIMITIVE);
+
+// Left state (kept in carry since the face below) and right state of window field i; carry takes
+// the left state of the face above.
+template <int STENCIL, int NW>
+__device__ __forceinline__ void shared_states(const double (&win)[NW][5], int i, const Params& prm, double& carry,
+                                              double& L, double& R) {
+    L = carry;
+    weno5_cell<STENCIL>(win[1][i], win[2][i], win[3][i], win[4][i], win[5][i], prm.eps_z, prm.eps_js, R, carry);
+}
+
+// Left states of the window's face, for the first face of a walk.
+template <int AXIS, int VAR, int STENCIL>
+__device__ __forceinline__ void carry_start(const double (&win)[Win<STENCIL>::n][5], const Params& prm,
+                                            double carry[5]) {
+    if constexpr (VAR == JFA_PRIMITIVE) {
+#pragma unroll
+        for (int i = 0; i < 5; ++i)
+            carry[i] = weno5<STENCIL>(win[0][i], win[1][i], win[2][i], win[3][i], win[4][i], prm.eps_z, prm.eps_js);
+    } else {
+        constexpr int m[2] = {Ax<AXIS>::m0, Ax<AXIS>::m1};
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            carry[i] = weno5<STENCIL>(win[0][m[i]], win[1][m[i]], win[2][m[i]], win[3][m[i]], win[4][m[i]], prm.eps_z,
+                                      prm.eps_js);
+    }
+}
+
+// Scaled characteristics of the primitives at a face's frozen state (eigendecomposition.py:425-431,
+// 517-521).  The reference's x0, x4 = k2 p -+ k1 u_n (k1 = 1/(2c), k2 = 1/(2 c^2 rho)) are
+// reconstructed as y = x / k1 = m p -+ u_n with m = 1/(rho c): one fma per cell, and m is the
+// frozen state's own inverse square root.  WENO is homogeneous, so the states scale back exactly
+// once the epsilon of the indicators is scaled alike (by 1/k1^2, WENO-JS by 1/k1^4).
+struct CharScale {
+    double m, k3, h0, h4, eps_z, eps_js;
+    __device__ __forceinline__ CharScale(const Frozen& f, const Params& prm) {
+        m = f.m;
+        k3 = f.inv_c * f.inv_c;
+        h0 = 0.5 * f.P[0] * f.inv_c;  // rho k1, of W_rho = rho (x0 + x4) + x1
+        h4 = 0.5 * f.P[0] * f.c;      // c^2 rho k1, of W_p = c^2 rho (x0 + x4)
+        const double s = 4.0 * (f.c * f.c);
+        eps_z = prm.eps_z * s;
+        eps_js = prm.eps_js * (s * s);
+    }
+    template <int v, int m0, int m1>
+    __device__ __forceinline__ void primitives(const double y[5], double W[5]) const {
+        const double s = y[0] + y[4];
+        W[0] = fma(h0, s, y[1]);
+        W[v] = 0.5 * (y[4] - y[0]);
+        W[m0] = y[2];
+        W[m1] = y[3];
+        W[4] = h4 * s;
+    }
+};
+
 // Face states WL, WR, UL, UR of one face from its six-cell window (primitives for PRIMITIVE and
 // CHAR-PRIMITIVE, conservatives otherwise); wl, wr are the primitives of the face's two cells,
 // read for CHAR-CONSERVATIVE.  The positivity limiter is applied by the callers (limit_side).
-template <int AXIS, int VAR, int STENCIL>
+//
+// CARRY (kCarry<VAR, STENCIL> schemes): the caller walks consecutive faces upwards.  The fields that
+// are reconstructed as they are stored (all primitives of PRIMITIVE, the two tangential velocities of
+// CHAR-PRIMITIVE) then take their left state from carry[], which holds it since the face below, and
+// leave the one of the face above there (carry_start fills it before the first face); cell 0 of the
+// window is not read for them.
+template <int AXIS, int VAR, int STENCIL, bool CARRY = false>
 __device__ __forceinline__ void face_states(const double (&win)[Win<STENCIL>::n][5], const double wl[5],
                                             const double wr[5], const Params& prm, double WL[5], double WR[5],
-                                            double UL[5], double UR[5]) {
+                                            double UL[5], double UR[5], double* carry = nullptr) {
     constexpr int v = Ax<AXIS>::v, m0 = Ax<AXIS>::m0, m1 = Ax<AXIS>::m1;
     constexpr int NW = Win<STENCIL>::n, H = Win<STENCIL>::h;
     if constexpr (VAR == JFA_PRIMITIVE || VAR == JFA_CONSERVATIVE) {
@@ -1114,11 +1222,15 @@ __device__ __forceinline__ void face_states(const double (&win)[Win<STENCIL>::n]
         double* QR = VAR == JFA_PRIMITIVE ? WR : UR;
 #pragma unroll
         for (int i = 0; i < 5; ++i) {
-            // WENO5Base slices j=0: cells -3..1, j=1: cells 2..-2 (weno5_base.py:30)
-            double cw[NW];
+            if constexpr (CARRY) {
+                shared_states<STENCIL, NW>(win, i, prm, carry[i], QL[i], QR[i]);
+            } else {
+                // WENO5Base slices j=0: cells -3..1, j=1: cells 2..-2 (weno5_base.py:30)
+                double cw[NW];
 #pragma unroll
-            for (int k = 0; k < NW; ++k) cw[k] = win[k][i];
-            recon_pair<STENCIL>(cw, prm, prm.dx2[AXIS], QL[i], QR[i]);
+                for (int k = 0; k < NW; ++k) cw[k] = win[k][i];
+                recon_pair<STENCIL>(cw, prm, prm.dx2[AXIS], QL[i], QR[i]);
+            }
         }
         if constexpr (VAR == JFA_PRIMITIVE) {
             cons_from_prim(WL, prm, UL);  // :279-280
@@ -1131,41 +1243,67 @@ __device__ __forceinline__ void face_states(const double (&win)[Win<STENCIL>::n]
         // frozen state from the cells left/right of the face (eigendecomposition.py:139-140)
         Frozen f;
         frozen_state<false>(win[H - 1], win[H], prm, f);
-        // get_characteristics_from_primitives (eigendecomposition.py:425-431):
-        // k1 = 0.5/c, k2 = 0.5/(c^2 rho), k3 = 1/c^2
-        const double k1 = 0.5 * f.inv_c;
-        const double k3 = f.inv_c * f.inv_c;
-        const double k2 = 0.5 * rcp1(f.rcc);
-        // one characteristic field at a time (x0 = k2 p - k1 u_n, x1 = rho - k3 p,
-        // x2, x3 = tangential velocities, x4 = k2 p + k1 u_n), each reconstructed L and R
         double cLv[5], cRv[5], t[NW];
+        if constexpr (STENCIL == JFA_WENO5_JS || STENCIL == JFA_WENO5_Z) {
+            const CharScale cs(f, prm);
 #pragma unroll
-        for (int k = 0; k < NW; ++k) t[k] = k2 * win[k][4] - k1 * win[k][v];
-        recon_pair<STENCIL>(t, prm, prm.dx2[AXIS], cLv[0], cRv[0]);
+            for (int k = 0; k < NW; ++k) t[k] = fma(cs.m, win[k][4], -win[k][v]);
+            weno5_pair<STENCIL>(t, cs.eps_z, cs.eps_js, cLv[0], cRv[0]);
 #pragma unroll
-        for (int k = 0; k < NW; ++k) t[k] = win[k][0] - k3 * win[k][4];
-        recon_pair<STENCIL>(t, prm, prm.dx2[AXIS], cLv[1], cRv[1]);
+            for (int k = 0; k < NW; ++k) t[k] = fma(cs.m, win[k][4], win[k][v]);
+            weno5_pair<STENCIL>(t, cs.eps_z, cs.eps_js, cLv[4], cRv[4]);
 #pragma unroll
-        for (int k = 0; k < NW; ++k) t[k] = win[k][m0];
-        recon_pair<STENCIL>(t, prm, prm.dx2[AXIS], cLv[2], cRv[2]);
+            for (int k = 0; k < NW; ++k) t[k] = fma(-cs.k3, win[k][4], win[k][0]);
+            weno5_pair<STENCIL>(t, prm.eps_z, prm.eps_js, cLv[1], cRv[1]);
+            if constexpr (CARRY) {
+                shared_states<STENCIL, NW>(win, m0, prm, carry[0], cLv[2], cRv[2]);
+                shared_states<STENCIL, NW>(win, m1, prm, carry[1], cLv[3], cRv[3]);
+            } else {
 #pragma unroll
-        for (int k = 0; k < NW; ++k) t[k] = win[k][m1];
-        recon_pair<STENCIL>(t, prm, prm.dx2[AXIS], cLv[3], cRv[3]);
+                for (int k = 0; k < NW; ++k) t[k] = win[k][m0];
+                weno5_pair<STENCIL>(t, prm.eps_z, prm.eps_js, cLv[2], cRv[2]);
 #pragma unroll
-        for (int k = 0; k < NW; ++k) t[k] = k2 * win[k][4] + k1 * win[k][v];
-        recon_pair<STENCIL>(t, prm, prm.dx2[AXIS], cLv[4], cRv[4]);
-        // get_primitives_from_characteristics (eigendecomposition.py:517-521)
-        const double sL = cLv[0] + cLv[4], sR = cRv[0] + cRv[4];
-        WL[0] = f.P[0] * sL + cLv[1];
-        WL[v] = f.c * (cLv[4] - cLv[0]);
-        WL[m0] = cLv[2];
-        WL[m1] = cLv[3];
-        WL[4] = f.rcc * sL;
-        WR[0] = f.P[0] * sR + cRv[1];
-        WR[v] = f.c * (cRv[4] - cRv[0]);
-        WR[m0] = cRv[2];
-        WR[m1] = cRv[3];
-        WR[4] = f.rcc * sR;
+                for (int k = 0; k < NW; ++k) t[k] = win[k][m1];
+                weno5_pair<STENCIL>(t, prm.eps_z, prm.eps_js, cLv[3], cRv[3]);
+            }
+            cs.primitives<v, m0, m1>(cLv, WL);
+            cs.primitives<v, m0, m1>(cRv, WR);
+        } else {
+            // get_characteristics_from_primitives (eigendecomposition.py:425-431):
+            // k1 = 0.5/c, k2 = 0.5/(c^2 rho), k3 = 1/c^2
+            const double k1 = 0.5 * f.inv_c;
+            const double k3 = f.inv_c * f.inv_c;
+            const double k2 = 0.5 * rcp1(f.rcc);
+            // one characteristic field at a time (x0 = k2 p - k1 u_n, x1 = rho - k3 p,
+            // x2, x3 = tangential velocities, x4 = k2 p + k1 u_n), each reconstructed L and R
+#pragma unroll
+            for (int k = 0; k < NW; ++k) t[k] = k2 * win[k][4] - k1 * win[k][v];
+            recon_pair<STENCIL>(t, prm, prm.dx2[AXIS], cLv[0], cRv[0]);
+#pragma unroll
+            for (int k = 0; k < NW; ++k) t[k] = win[k][0] - k3 * win[k][4];
+            recon_pair<STENCIL>(t, prm, prm.dx2[AXIS], cLv[1], cRv[1]);
+#pragma unroll
+            for (int k = 0; k < NW; ++k) t[k] = win[k][m0];
+            recon_pair<STENCIL>(t, prm, prm.dx2[AXIS], cLv[2], cRv[2]);
+#pragma unroll
+            for (int k = 0; k < NW; ++k) t[k] = win[k][m1];
+            recon_pair<STENCIL>(t, prm, prm.dx2[AXIS], cLv[3], cRv[3]);
+#pragma unroll
+            for (int k = 0; k < NW; ++k) t[k] = k2 * win[k][4] + k1 * win[k][v];
+            recon_pair<STENCIL>(t, prm, prm.dx2[AXIS], cLv[4], cRv[4]);
+            // get_primitives_from_characteristics (eigendecomposition.py:517-521)
+            const double sL = cLv[0] + cLv[4], sR = cRv[0] + cRv[4];
+            WL[0] = f.P[0] * sL + cLv[1];
+            WL[v] = f.c * (cLv[4] - cLv[0]);
+            WL[m0] = cLv[2];
+            WL[m1] = cLv[3];
+            WL[4] = f.rcc * sL;
+            WR[0] = f.P[0] * sR + cRv[1];
+            WR[v] = f.c * (cRv[4] - cRv[0]);
+            WR[m0] = cRv[2];
+            WR[m1] = cRv[3];
+            WR[4] = f.rcc * sR;
+        }
         cons_from_prim(WL, prm, UL);  // :401-402
         cons_from_prim(WR, prm, UR);
     } else {  // CHAR-CONSERVATIVE (:404-417)

@@ -24,17 +24,24 @@
 namespace jfa {
 
 constexpr int kInnerBlock = 256;
-constexpr int kMarchBlockMax = 256;
+constexpr int kMarchBlock = 256;
 
 // Face flux from a register window (cell k-h relative to the cell right of the face, k < n; 6 cells,
 // 8 for WENO7-JS).
 // CHAR-CONSERVATIVE also needs the primitives of the two cells adjacent to the face.
-template <class T, int AXIS, int VAR, int STENCIL, int RIEMANN, bool FLIM>
+// CARRY: face_states' states shared by consecutive faces, in carry.  after_states runs once the
+// window's lowest cell is no longer needed.
+struct Nothing {
+    __device__ __forceinline__ void operator()() const {}
+};
+template <class T, int AXIS, int VAR, int STENCIL, int RIEMANN, bool FLIM, bool CARRY = false, class After = Nothing>
 __device__ __forceinline__ void window_flux(const double (&win)[Win<STENCIL>::n][5], const T* __restrict__ W,
                                             const T* __restrict__ U, int64_t b_right, int64_t sa, int64_t fs,
-                                            const Params& prm, double F[5]) {
+                                            const Params& prm, double F[5], double* carry = nullptr,
+                                            After after_states = After()) {
     if constexpr (RIEMANN == kFluxSplit) {
         flux_split_face<AXIS, STENCIL>(win, prm, F);
+        after_states();
     } else {
         double wl[5], wr[5];
         if constexpr (VAR == JFA_CHAR_CONSERVATIVE) {
@@ -45,7 +52,8 @@ __device__ __forceinline__ void window_flux(const double (&win)[Win<STENCIL>::n]
             }
         }
         double WL[5], WR[5], UL[5], UR[5];
-        face_states<AXIS, VAR, STENCIL>(win, wl, wr, prm, WL, WR, UL, UR);
+        face_states<AXIS, VAR, STENCIL, CARRY>(win, wl, wr, prm, WL, WR, UL, UR, carry);
+        after_states();
         if (prm.limiter) {
             double c[5];
 #pragma unroll
@@ -55,7 +63,7 @@ __device__ __forceinline__ void window_flux(const double (&win)[Win<STENCIL>::n]
             for (int i = 0; i < 5; ++i) c[i] = ld(W, i * fs + b_right);
             limit_side<VAR>(c, prm, WR, UR);
         }
-        riemann<AXIS, RIEMANN>(WL, WR, UL, UR, prm, F);
+        riemann<AXIS, RIEMANN, VAR == JFA_PRIMITIVE || VAR == JFA_CHAR_PRIMITIVE>(WL, WR, UL, UR, prm, F);
     }
     if constexpr (FLIM) {  // positivity flux limiter, with the step's dt (space_solver.py:530-541)
         double wl_[5], wr_[5], ul_[5], ur_[5];
@@ -72,70 +80,101 @@ __device__ __forceinline__ void window_flux(const double (&win)[Win<STENCIL>::n]
 }
 
 // ------------------------------------------------------------------ MARCH kernel
-// grid: x over IN (lanes), y over the third axis O, z over chunks of L cells along A.
-// The plain convective variants are held to 3 waves per SIMD (168 VGPRs; they need 162): one
-// register more costs a third of the resident waves of this VALU-bound loop.
+// Lanes run over the columns along A in buffer order, rows of IN after one another (a row of 65
+// columns costs 65 lanes, not 128); grid.y runs over chunks of L cells along A.
+// Addresses are a wave-uniform base (the wave's first column; scalar registers) and one 32-bit lane
+// offset; where a wave's rows lie too far apart for it, rowlen is the row rounded up to whole waves
+// (packs_rows).
+// Bound: FP64 issue (520 FP64 instructions a face with the WENO5 stencils) and, for the loads and
+// stores that this must hide, latency: the next cell and the RHS of the step are loaded a whole face
+// ahead, before the step's stores, so no wait covers a store (256^3 CHAR-PRIMITIVE WENO5-Z HLLC, us
+// per sweep along x / y: 507 / 589 loading at the top of the step, 433 / 476 ahead).  The plain
+// convective variants are held to two waves per SIMD so that nothing spills.  The others need the registers: with the
+// loads ahead the dissipative variants fall to one wave per SIMD (128^3 viscous PRIMITIVE, us per
+// stage: 474 ahead, 388 at the top of the step).
+template <int VAR, int RIEMANN, bool DISS, bool FLIM>
+constexpr bool kPlainMarch = !(DISS || FLIM || VAR == JFA_CHAR_CONSERVATIVE || RIEMANN == kFluxSplit);
+
 template <class T, int A, int IN, int VAR, int STENCIL, int RIEMANN, bool DISS, bool FLIM>
-__global__ __launch_bounds__(kMarchBlockMax)
-JFA_WAVES_PER_EU((DISS || FLIM || VAR == JFA_CHAR_CONSERVATIVE || RIEMANN == kFluxSplit) ? 1 : 3) void march_kernel(
-    const T* __restrict__ W, const T* __restrict__ U, Geo G, Params prm, int L, int accumulate,
+__global__ __launch_bounds__(kMarchBlock)
+JFA_WAVES_PER_EU((kPlainMarch<VAR, RIEMANN, DISS, FLIM> ? 2 : 1)) void march_kernel(
+    const T* __restrict__ W, const T* __restrict__ U, Geo G, Params prm, int L, int rowlen, int accumulate,
     double* __restrict__ R) {
     constexpr int O = 3 - A - IN;
-    const int iin = blockIdx.x * blockDim.x + threadIdx.x;
-    if (iin >= G.n[IN]) return;  // no barriers in this kernel
-    const int io = blockIdx.y;
-    const int a0 = blockIdx.z * L;
+    const int c0 = uni((int)(blockIdx.x * kMarchBlock + (threadIdx.x & ~63u)));  // the wave's first column
+    const int io0 = c0 / rowlen, iin0 = c0 - io0 * rowlen;
+    int io = io0, iin = iin0 + (int)(threadIdx.x & 63);
+    if (iin >= rowlen) {
+        io += iin / rowlen;
+        iin = iin % rowlen;
+    }
+    if (io >= G.n[O] || iin >= G.n[IN]) return;  // no barriers in this kernel
+    const int a0 = blockIdx.y * L;
     const int a1 = min(a0 + L, G.n[A]);
     const int64_t sa = G.s[A];
     const int64_t fs = G.fs;
-    // buffer index of the column's cell with interior index 0 along A
-    const int64_t bcol = (int64_t)(io + G.off[O]) * G.s[O] + (int64_t)(iin + G.off[IN]) * G.s[IN] +
-                         (int64_t)G.off[A] * sa;
+    // buffer index of the cell with interior index 0 along A: wave-uniform part (row io0) and lane part
+    const int64_t bcol = (int64_t)(io0 + G.off[O]) * G.s[O] + G.off[IN] + (int64_t)G.off[A] * sa;
+    const int64_t bl = (int64_t)(io - io0) * G.s[O] + iin;
+    const uint32_t voff = (uint32_t)bl * (uint32_t)sizeof(T);
     constexpr bool cons_win = (VAR == JFA_CONSERVATIVE || VAR == JFA_CHAR_CONSERVATIVE);
     constexpr int NW = Win<STENCIL>::n, H = Win<STENCIL>::h;
     const T* __restrict__ src = cons_win ? U : W;
-    double win[NW][5];
+    constexpr bool CARRY = RIEMANN != kFluxSplit && kCarry<VAR, STENCIL>;
+    constexpr bool AHEAD = kPlainMarch<VAR, RIEMANN, DISS, FLIM>;
+    double win[NW][5], nxt[5], carry[5];
 #pragma unroll
     for (int k = 0; k < NW; ++k)
 #pragma unroll
-        for (int i = 0; i < 5; ++i) win[k][i] = ld(src, i * fs + bcol + (int64_t)(a0 - H + k) * sa);
+        for (int i = 0; i < 5; ++i) win[k][i] = ldo(src + (i * fs + bcol + (int64_t)(a0 - H + k) * sa), voff);
+#pragma unroll
+    for (int i = 0; i < 5; ++i)
+        if (AHEAD) nxt[i] = ldo(src + (i * fs + bcol + (int64_t)(a0 + H) * sa), voff);
+    if constexpr (CARRY) carry_start<A, VAR, STENCIL>(win, prm, carry);
     double Fp[5];
-    window_flux<T, A, VAR, STENCIL, RIEMANN, FLIM>(win, W, U, bcol + (int64_t)a0 * sa, sa, fs, prm, Fp);
+    window_flux<T, A, VAR, STENCIL, RIEMANN, FLIM, CARRY>(win, W, U, bl + bcol + (int64_t)a0 * sa, sa, fs, prm, Fp, carry);
     int cr[3];  // right cell of the current face (dissipative fluxes)
     cr[A] = a0;
     cr[O] = io;
     cr[IN] = iin;
     if constexpr (DISS) dissipative_face<T, A>(W, G, prm, cr, Fp);
     // R layout (5, N0, N1, N2)
-    int c[3];
-    c[A] = a0;
-    c[O] = io;
-    c[IN] = iin;
     const int64_t ncell = (int64_t)G.n[0] * G.n[1] * G.n[2];
-    int64_t r = ((int64_t)c[0] * G.n[1] + c[1]) * G.n[2] + c[2];
-    const int64_t rs = A == 0 ? (int64_t)G.n[1] * G.n[2] : (A == 1 ? (int64_t)G.n[2] : 1);
+    const int64_t rsA = A == 0 ? (int64_t)G.n[1] * G.n[2] : (A == 1 ? (int64_t)G.n[2] : 1);
+    const int64_t rsO = O == 0 ? (int64_t)G.n[1] * G.n[2] : (O == 1 ? (int64_t)G.n[2] : 1);
+    int64_t r = (int64_t)io0 * rsO + (int64_t)a0 * rsA;
+    const uint32_t roff = (uint32_t)((int64_t)(io - io0) * rsO + iin) * (uint32_t)sizeof(double);
     const double odx = G.one_dx[A];
-    // The new cell of the window is loaded at the top of its step, not a step ahead: the five
-    // registers of a prefetch push the plain variants past 168 VGPRs into spills, which cost
-    // more than the load latency that three resident waves already cover.
-    for (int a = a0; a < a1; ++a, r += rs) {
+    for (int a = a0; a < a1; ++a, r += rsA) {
+        uint32_t vo = voff, ro = roff;
+        JFA_OPAQUE(vo);  // keeps per-tap addresses from being hoisted out of the loop
+        JFA_OPAQUE(ro);
 #pragma unroll
         for (int k = 0; k < NW - 1; ++k)
 #pragma unroll
             for (int i = 0; i < 5; ++i) win[k][i] = win[k + 1][i];
 #pragma unroll
-        for (int i = 0; i < 5; ++i) win[NW - 1][i] = ld(src, i * fs + bcol + (int64_t)(a + H) * sa);
+        for (int i = 0; i < 5; ++i)
+            win[NW - 1][i] = AHEAD ? nxt[i] : ldo(src + (i * fs + bcol + (int64_t)(a + H) * sa), vo);
+        // the next step's cell (the last step repeats its own) and this step's RHS
+        const int64_t bn = bcol + (int64_t)(a + 1 < a1 ? a + 1 + H : a + H) * sa;
+        double rr[5];
+#pragma unroll
+        for (int i = 0; i < 5; ++i)
+            if (AHEAD) nxt[i] = ldo(src + (i * fs + bn), vo);
+#pragma unroll
+        for (int i = 0; i < 5; ++i) rr[i] = accumulate ? ldo(R + (i * ncell + r), ro) : 0.0;
+        JFA_SCHED_BARRIER();
         double Fn[5];
-        window_flux<T, A, VAR, STENCIL, RIEMANN, FLIM>(win, W, U, bcol + (int64_t)(a + 1) * sa, sa, fs, prm, Fn);
+        window_flux<T, A, VAR, STENCIL, RIEMANN, FLIM, CARRY>(win, W, U, bl + bcol + (int64_t)(a + 1) * sa, sa, fs, prm,
+                                                              Fn, carry);
         if constexpr (DISS) {
             cr[A] = a + 1;
             dissipative_face<T, A>(W, G, prm, cr, Fn);
         }
 #pragma unroll
         for (int i = 0; i < 5; ++i) {
-            const double d = odx * (Fp[i] - Fn[i]);  // space_solver.py:597-599
-            double* p = R + i * ncell + r;
-            *p = accumulate ? *p + d : 0.0 + d;
+            sto(R + (i * ncell + r), ro, rr[i] + odx * (Fp[i] - Fn[i]));  // space_solver.py:597-599
             Fp[i] = Fn[i];
         }
     }
@@ -342,18 +381,31 @@ static inline int64_t inner_blocks(const Geo& G) {
     return (nwaves + (kInnerBlock / 64) - 1) / (kInnerBlock / 64);
 }
 
-// Chunk length L along A: every wave marches L cells (L+1 faces).  The waves of one launch
-// run in ceil(waves / slots) rounds, slots = CUs x resident waves per CU of this kernel, so
-// L is chosen to minimise rounds x (L + 1) -- short chunks cost an extra face each, a
-// part-filled last round idles the chip.  waves_per_layer: wavefronts of one chunk layer.
-static inline int march_chunk(int nA, int64_t waves_per_layer, int64_t slots) {
-    int best_L = 4;
+// Time of `waves` equal wavefronts on `simds` SIMDs that hold `slots` of them, in units of a wavefront
+// alone on its SIMD: one wave issues 60 % of what the SIMD can (its FP64 instructions depend on one
+// another), so k waves of a SIMD take max(1, 0.85 k) (measured on the 2-D sweeps), and a partly
+// filled last round lasts as its fullest SIMD.
+static inline double rounds_time(int64_t waves, int64_t slots, int64_t simds) {
+    auto t = [](int64_t k) { return k > 1 ? 0.85 * (double)k : 1.0; };
+    const int64_t full = waves / slots, rem = waves % slots;
+    return (double)full * t((slots + simds - 1) / simds) + (rem ? t((rem + simds - 1) / simds) : 0.0);
+}
+
+// Whether 64 consecutive positions of rows of `len` positions, axis O apart, lie within 32-bit byte
+// offsets of the first row.
+template <class T>
+static inline bool packs_rows(const Geo& G, int O, int len) {
+    return (int64_t)(64 / len + 1) * G.s[O] * (int64_t)sizeof(T) < (int64_t)1 << 31;
+}
+
+// Chunk length L along A: every wave marches L cells (L + 1 faces); short chunks cost an extra face
+// each, a part-filled last round idles the chip.  layer: wavefronts of one chunk layer.
+static inline int march_chunk(int nA, int64_t layer, int64_t slots, int64_t simds) {
+    int best_L = 1;
     double best = 1e300;
-    for (int L = 4; L <= 64; ++L) {
+    for (int L = 1; L <= 64; ++L) {
         const int64_t chunks = ((int64_t)nA + L - 1) / L;
-        const int64_t waves = chunks * waves_per_layer;
-        const int64_t rounds = (waves + slots - 1) / slots;
-        const double cost = (double)rounds * (L + 1);
+        const double cost = rounds_time(chunks * layer, slots, simds) * (L + 1);
         if (cost < best * 0.999) {
             best = cost;
             best_L = L;
@@ -363,8 +415,7 @@ static inline int march_chunk(int nA, int64_t waves_per_layer, int64_t slots) {
     return best_L;
 }
 
-// resident waves of a kernel on the whole device (cached per kernel instance)
-static inline int64_t device_wave_slots(const void* kernel, int block) {
+static inline int64_t device_cus() {
     static int num_cu = 0;
     if (num_cu == 0) {
         int dev = 0;
@@ -372,25 +423,30 @@ static inline int64_t device_wave_slots(const void* kernel, int block) {
             hipDeviceGetAttribute(&num_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || num_cu <= 0)
             num_cu = 256;
     }
+    return num_cu;
+}
+
+// resident waves of a kernel on the whole device (cached per kernel instance)
+static inline int64_t device_wave_slots(const void* kernel, int block) {
     int blocks = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, block, 0) != hipSuccess || blocks <= 0)
         blocks = 1;
-    return (int64_t)num_cu * blocks * ((block + 63) / 64);
+    return device_cus() * blocks * ((block + 63) / 64);
 }
 
 template <class T, int A, int IN, int VAR, int STENCIL, int RIEMANN, bool DISS, bool FLIM>
 static void launch_march(const void* W, const void* U, const Geo& G, const Params& prm, int accumulate, double* R,
                          hipStream_t st) {
     constexpr int O = 3 - A - IN;
-    int bx = ((G.n[IN] + 63) / 64) * 64;
-    if (bx > kMarchBlockMax) bx = kMarchBlockMax;
-    static int64_t slots[kMarchBlockMax / 64 + 1] = {0};
-    int64_t& sl = slots[bx / 64];
-    if (sl == 0) sl = device_wave_slots((const void*)march_kernel<T, A, IN, VAR, STENCIL, RIEMANN, DISS, FLIM>, bx);
-    const int L = march_chunk(G.n[A], ((int64_t)G.n[IN] + 63) / 64 * G.n[O], sl);
-    dim3 grid((unsigned)((G.n[IN] + bx - 1) / bx), (unsigned)G.n[O], (unsigned)((G.n[A] + L - 1) / L));
-    hipLaunchKernelGGL((march_kernel<T, A, IN, VAR, STENCIL, RIEMANN, DISS, FLIM>), grid, dim3(bx), 0, st,
-                       static_cast<const T*>(W), static_cast<const T*>(U), G, prm, L, accumulate, R);
+    static int64_t slots = 0;
+    if (slots == 0)
+        slots = device_wave_slots((const void*)march_kernel<T, A, IN, VAR, STENCIL, RIEMANN, DISS, FLIM>, kMarchBlock);
+    const int rowlen = packs_rows<T>(G, O, G.n[IN]) ? G.n[IN] : (G.n[IN] + 63) / 64 * 64;
+    const int64_t cols = (int64_t)rowlen * G.n[O];
+    const int L = march_chunk(G.n[A], (cols + 63) / 64, slots, 4 * device_cus());
+    dim3 grid((unsigned)((cols + kMarchBlock - 1) / kMarchBlock), (unsigned)((G.n[A] + L - 1) / L));
+    hipLaunchKernelGGL((march_kernel<T, A, IN, VAR, STENCIL, RIEMANN, DISS, FLIM>), grid, dim3(kMarchBlock), 0, st,
+                       static_cast<const T*>(W), static_cast<const T*>(U), G, prm, L, rowlen, accumulate, R);
 }
 
 template <class T, int IN, int VAR, int STENCIL, int RIEMANN, bool DISS, bool FLIM>
