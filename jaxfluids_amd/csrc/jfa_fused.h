@@ -13,9 +13,11 @@
 // finishes the stage for its cell: U = c0 U + c1 U_n + dt m rhs (RK3.py:27-62),
 // W = prim(U), stores both, scatters the cell into the halo positions the face-halo
 // fill copies it to (U halo = cons(W halo), outer/material.py:248-250), and reduces the
-// CFL wave speed of the new state into one partial per block.
+// CFL wave speed of the new state into one partial per block.  For the common schemes
+// (kFinal) the FINAL kernel takes the place of the last MARCH and of INNER: it walks along
+// the last A and evaluates both axes' faces and the finish of each row on the way.
 //
-// Included by the per-storage-type translation units jfa_fused_f64.hip / _f32.hip.
+// Included by the jfa_fused_<variable>.hip and _f64.hip / _f32.hip translation units.
 #pragma once
 
 #include "jfa_common.h"
@@ -79,6 +81,15 @@ __device__ __forceinline__ void window_flux(const double (&win)[Win<STENCIL>::n]
     }
 }
 
+// The options most simulations run with, as constants: kernels compiled for them drop the run-time
+// switches and the scalar registers these hold.
+__device__ __forceinline__ Params common_options(Params p) {
+    p.signal_speed = JFA_SS_EINFELDT;
+    p.frozen = JFA_FROZEN_ARITHMETIC;
+    p.limiter = 0;
+    return p;
+}
+
 // ------------------------------------------------------------------ MARCH kernel
 // Lanes run over the columns along A in buffer order, rows of IN after one another (a row of 65
 // columns costs 65 lanes, not 128); grid.y runs over chunks of L cells along A.
@@ -88,19 +99,21 @@ __device__ __forceinline__ void window_flux(const double (&win)[Win<STENCIL>::n]
 // Bound: FP64 issue (520 FP64 instructions a face with the WENO5 stencils) and, for the loads and
 // stores that this must hide, latency: the next cell and the RHS of the step are loaded a whole face
 // ahead, before the step's stores, so no wait covers a store (256^3 CHAR-PRIMITIVE WENO5-Z HLLC, us
-// per sweep along x / y: 507 / 589 loading at the top of the step, 433 / 476 ahead).  The plain
-// convective variants are held to two waves per SIMD so that nothing spills.  The others need the registers: with the
+// per sweep along x / y: 507 / 589 loading at the top of the step, 433 / 476 ahead, 397 / - with the
+// common options as constants).  The plain convective variants are held to two waves per SIMD so that
+// nothing spills; the common ones fit three by themselves.  The others need the registers: with the
 // loads ahead the dissipative variants fall to one wave per SIMD (128^3 viscous PRIMITIVE, us per
 // stage: 474 ahead, 388 at the top of the step).
 template <int VAR, int RIEMANN, bool DISS, bool FLIM>
 constexpr bool kPlainMarch = !(DISS || FLIM || VAR == JFA_CHAR_CONSERVATIVE || RIEMANN == kFluxSplit);
 
-template <class T, int A, int IN, int VAR, int STENCIL, int RIEMANN, bool DISS, bool FLIM>
+template <class T, int A, int IN, int VAR, int STENCIL, int RIEMANN, bool DISS, bool FLIM, bool COMMON>
 __global__ __launch_bounds__(kMarchBlock)
 JFA_WAVES_PER_EU((kPlainMarch<VAR, RIEMANN, DISS, FLIM> ? 2 : 1)) void march_kernel(
-    const T* __restrict__ W, const T* __restrict__ U, Geo G, Params prm, int L, int rowlen, int accumulate,
+    const T* __restrict__ W, const T* __restrict__ U, Geo G, Params prm_, int L, int rowlen, int accumulate,
     double* __restrict__ R) {
     constexpr int O = 3 - A - IN;
+    const Params prm = COMMON ? common_options(prm_) : prm_;
     const int c0 = uni((int)(blockIdx.x * kMarchBlock + (threadIdx.x & ~63u)));  // the wave's first column
     const int io0 = c0 / rowlen, iin0 = c0 - io0 * rowlen;
     int io = io0, iin = iin0 + (int)(threadIdx.x & 63);
@@ -343,6 +356,254 @@ __global__ __launch_bounds__(kInnerBlock) void inner_kernel(const T* __restrict_
     }
 }
 
+// ------------------------------------------------------------------ FINAL kernel
+// The last two sweeps of a stage and its finish in one pass (the common schemes, kFinal): along A,
+// the last active axis below IN, and along IN.  It takes the place of MARCH<A> + INNER and with them
+// of a write and two reads of the scratch RHS (a third of a 3-D stage's traffic; a 2-D stage needs no
+// scratch RHS at all), and of every re-read of a face window through the caches.
+//
+// A wavefront holds 64 consecutive cells of rows along IN and walks along A.  Rows live in LDS, NW - 1
+// of them in a ring (5 fields each): the A window of a lane is its own column of the ring, the IN
+// window of the row that is finished is the row beside the lane's cell, so every cell is loaded from
+// memory once (plus H rows per chunk).  How rows are cut (lane_map):
+//   packed = 0: each wave takes 64 cells of one row; five cells beside them are loaded as well, and
+//     the flux above its last cell is evaluated for all rows of the chunk before the walk (lane k: row
+//     a0 + k).  No lane idles where the row length is a multiple of 64.
+//   packed = 1: rows of N + 6 positions (with the windows' halo cells) after one another; a wave takes
+//     64 positions, of which the middle 58 have their whole window, and the next wave starts 58 on.
+//     For ragged rows: a row of 80 cells keeps 84 % of the lanes, against 62 %.
+// Loads run ahead: the finish's (scratch RHS, U, U_n) at the top of the row, two faces before their
+// use; the next row's during the A face, once the reconstruction is done with the window.
+//
+// Bound: FP64 issue at the clock the card holds under it (70 % of the cycles issue; 1.97 GHz), about
+// 240 VGPRs (two waves per SIMD; three spill), 2.5 GB read and 1.6 GB written per stage at 256^3.
+// Measured there (FP64, sustained, us per stage with the x sweep): CHAR-PRIMITIVE WENO5-Z HLLC 2000
+// with MARCH + INNER, 1460 with this kernel (windows through the caches instead of LDS 1680, the
+// finish's loads after the IN face 1490); PRIMITIVE WENO5-JS 1770 and 1425.  256 x 256: 22.8 and
+// 12.9, 65 x 64 x 63: 64 and 47 us.
+// The shared left states along A (CARRY) pay in CHAR-PRIMITIVE (1500 without); PRIMITIVE's five
+// spill (1860 against 1415).
+template <int VAR, int STENCIL, int RIEMANN, bool DISS, bool FLIM>
+constexpr bool kFinal = kCarry<VAR, STENCIL> && (RIEMANN == JFA_HLLC || RIEMANN == JFA_RUSANOV) && !DISS && !FLIM;
+
+// The cut of the rows and the chunks of FINAL, chosen on the host (final_plan).
+struct FinalPlan {
+    int packed;
+    int L;       // cells of a chunk along A, <= 64
+    int layer;   // wavefronts of one chunk layer
+    int waves;   // layer x chunks
+};
+constexpr int kPackStep = 58;  // positions a packed wave advances: 64 less the window's reach (3 + 2) and the upper face
+
+template <class T, int A, int IN, int VAR, int STENCIL, int RIEMANN>
+__global__ __launch_bounds__(kInnerBlock) JFA_WAVES_PER_EU(2) void final_kernel(const T* __restrict__ W,
+                                                                                const T* __restrict__ U, Geo G,
+                                                                                Params prm_, FinalPlan plan,
+                                                                                InnerArgs<T> args) {
+    constexpr int O = 3 - A - IN;
+    constexpr int NW = Win<STENCIL>::n, H = Win<STENCIL>::h;
+    constexpr int RW = 64 + NW - 1;  // cells of a row in LDS: H below the wave's first cell, H - 1 above the last
+    constexpr bool CARRY = VAR == JFA_CHAR_PRIMITIVE;
+    const Params prm = common_options(prm_);
+    __shared__ double rows[kInnerBlock / 64][NW - 1][5][RW + 3];
+    __shared__ double top[kInnerBlock / 64][5][64];
+    const int lane = threadIdx.x & 63;
+    const int wid = threadIdx.x >> 6;
+    const int wv = uni((int)(blockIdx.x * (kInnerBlock / 64) + (threadIdx.x >> 6)));
+    double vmax = 0.0;
+    if (wv < plan.waves) {  // whole wavefronts
+        const int chunk = wv / plan.layer;
+        const int w = wv - chunk * plan.layer;
+        const int N = G.n[IN];
+        // this lane's cell (f, the face below it; row io of axis O) and what it owns
+        int io0, io, f;
+        bool vcell;
+        if (plan.packed) {
+            const int P = N + NW;
+            const int g0 = w * kPackStep;
+            io0 = g0 / P;
+            const int j = g0 - io0 * P + lane;
+            io = io0 + j / P;
+            f = j % P - H;
+            vcell = lane >= H && lane < H + kPackStep && f >= 0 && f < N && io < G.n[O];
+            if (io >= G.n[O]) {  // past the last row: any valid cell
+                io = io0;
+                f = 0;
+            }
+        } else {
+            const int nseg = (N + 63) / 64;
+            io0 = io = w / nseg;
+            f = (w - io * nseg) * 64 + lane;
+            vcell = f < N;
+        }
+        const int fc = f < N + H - 1 ? f : N + H - 1;  // columns past the row read its last halo cell
+        const int64_t sa = G.s[A], fs = G.fs;
+        // wave-uniform part of the buffer index: H cells below the first of row io0, coordinate 0 along A
+        const int64_t brow = (int64_t)(io0 + G.off[O]) * G.s[O] + (int64_t)G.off[A] * sa + G.off[IN] - H;
+        const int bl = (io - io0) * (int)G.s[O] + fc + H;  // the lane's part
+        const uint32_t voff = (uint32_t)bl * (uint32_t)sizeof(T);
+        // lanes 0 .. NW - 2 also hold the row's cells beside the wave's 64: H below, H - 1 above (the
+        // other lanes repeat the last of them into the row's padding; packed waves do not read them)
+        const int f0 = plan.packed ? 0 : (w - io0 * ((N + 63) / 64)) * 64;
+        const int hl = lane < NW - 1 ? lane : NW - 2;
+        const int fh = hl < H ? f0 - H + hl : f0 + 64 + hl - H;
+        const uint32_t hoff = (uint32_t)((fh < N + H - 1 ? fh : N + H - 1) + H) * (uint32_t)sizeof(T);
+        const int hpos = lane < H ? lane : (lane < NW - 1 ? 64 + lane : RW);
+        double(*const my)[5][RW + 3] = rows[wid];
+        const int a0 = chunk * plan.L, a1 = min(a0 + plan.L, G.n[A]);
+        const int64_t ncell = (int64_t)G.n[0] * G.n[1] * G.n[2];
+        const int64_t rsA = A == 0 ? (int64_t)G.n[1] * G.n[2] : (int64_t)G.n[2];
+        const int64_t rsO = O == 0 ? (int64_t)G.n[1] * G.n[2] : (O == 1 ? (int64_t)G.n[2] : 1);
+        const int64_t r0 = (int64_t)io0 * rsO;
+        const uint32_t roff = vcell ? (uint32_t)((io - io0) * (int)rsO + f) * (uint32_t)sizeof(double) : 0u;
+
+        // upper face of the wave's last cell, for the row a0 + lane
+        if (!plan.packed && f0 + 64 <= N && lane < a1 - a0) {
+            const int64_t b = brow + (int64_t)a0 * sa + f0 + 64 + H;
+            const uint32_t v = (uint32_t)lane * (uint32_t)sa * (uint32_t)sizeof(T);
+            double win[NW][5], Ft[5];
+#pragma unroll
+            for (int k = 0; k < NW; ++k)
+#pragma unroll
+                for (int i = 0; i < 5; ++i) win[k][i] = ldo(W + (i * fs + b + (k - H)), v);
+            window_flux<T, IN, VAR, STENCIL, RIEMANN, false>(win, W, U, b + (int64_t)lane * sa, 1, fs, prm, Ft);
+#pragma unroll
+            for (int i = 0; i < 5; ++i) top[wid][i][lane] = Ft[i];
+        }
+        double carry[5], Fp[5], nxt[5], hal[5];
+        {
+            double win[NW][5];
+#pragma unroll
+            for (int k = 0; k < NW; ++k)
+#pragma unroll
+                for (int i = 0; i < 5; ++i) win[k][i] = ldo(W + (i * fs + brow + (int64_t)(a0 - H + k) * sa), voff);
+#pragma unroll
+            for (int k = 0; k < NW - 1; ++k)
+#pragma unroll
+                for (int i = 0; i < 5; ++i) my[k][i][H + lane] = win[k + 1][i];
+#pragma unroll
+            for (int k = H; k < NW; ++k)  // rows a0 .. a0 + H - 1
+#pragma unroll
+                for (int i = 0; i < 5; ++i)
+                    my[k - 1][i][hpos] = ldo(W + (i * fs + brow + (int64_t)(a0 - H + k) * sa), hoff);
+            if constexpr (CARRY) carry_start<A, VAR, STENCIL>(win, prm, carry);
+            window_flux<T, A, VAR, STENCIL, RIEMANN, false, CARRY>(win, W, U, bl + brow + (int64_t)a0 * sa, sa, fs, prm,
+                                                                   Fp, carry);
+        }
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+            nxt[i] = ldo(W + (i * fs + brow + (int64_t)(a0 + H) * sa), voff);
+            hal[i] = ldo(W + (i * fs + brow + (int64_t)(a0 + H) * sa), hoff);
+        }
+        double c0, c1, m;
+        rk3_coeffs(args.stage, c0, c1, m);
+        const double ts = args.mode == 0 ? 0.0 : (args.dt_dev ? args.dt_dev[0] : args.dt_host) * m;  // RK3.py:60
+        int slot = 0;  // ring position of row a - H + 1
+        for (int a = a0; a < a1; ++a) {
+            uint32_t vo = voff, ro = roff, ho = hoff;
+            JFA_OPAQUE(vo);
+            JFA_OPAQUE(ro);
+            JFA_OPAQUE(ho);
+            int64_t fso = fs;  // opaque: multiples of it are formed again, not kept in (spilled) scalar registers
+            JFA_OPAQUE_S(fso);
+            const int64_t rb = brow + (int64_t)a * sa;
+            const int64_t rr0 = r0 + a * rsA;
+            auto row = [&](int k) { return slot + k >= NW - 1 ? slot + k - (NW - 1) : slot + k; };
+            // what the finish of this row needs from memory, two faces ahead
+            double rr[5], ui[5], un[5];
+#pragma unroll
+            for (int i = 0; i < 5; ++i) {
+                rr[i] = args.accumulate ? ldo(args.R + (i * ncell + rr0), ro) : 0.0;
+                if (args.mode) {
+                    ui[i] = ldo(args.Uin + (i * fso + rb), vo);
+                    if (args.stage > 0) un[i] = ldo(args.Un + (i * fso + rb), vo);
+                }
+            }
+            JFA_SCHED_BARRIER();
+            JFA_WAVE_FENCE();
+            double dz[5];
+            {
+                double zw[NW][5], Fz[5];
+                const int q = row(H - 1);
+#pragma unroll
+                for (int k = 0; k < NW; ++k)
+#pragma unroll
+                    for (int i = 0; i < 5; ++i) zw[k][i] = my[q][i][lane + k];
+                window_flux<T, IN, VAR, STENCIL, RIEMANN, false>(zw, W, U, bl + rb, 1, fs, prm, Fz);
+#pragma unroll
+                for (int i = 0; i < 5; ++i) {
+                    const double e = top[wid][i][a - a0];
+                    const double up = __shfl_down(Fz[i], 1, 64);
+                    dz[i] = G.one_dx[IN] * (Fz[i] - (lane == 63 ? e : up));
+                }
+            }
+            JFA_WAVE_FENCE();
+            double Fn[5];
+            {
+                double win[NW][5];
+#pragma unroll
+                for (int k = 0; k < NW - 1; ++k) {
+                    const int q = row(k);
+#pragma unroll
+                    for (int i = 0; i < 5; ++i) win[k][i] = my[q][i][H + lane];
+                }
+#pragma unroll
+                for (int i = 0; i < 5; ++i) win[NW - 1][i] = nxt[i];
+                const int64_t nb = rb + (a + 1 < a1 ? H + 1 : H) * sa;
+                window_flux<T, A, VAR, STENCIL, RIEMANN, false, CARRY>(
+                    win, W, U, bl + rb + sa, sa, fs, prm, Fn, carry, [&]() {
+                        // the new row takes the place of the lowest; the next one is loaded ahead (the
+                        // last step repeats its own)
+#pragma unroll
+                        for (int i = 0; i < 5; ++i) {
+                            my[slot][i][H + lane] = nxt[i];
+                            my[slot][i][hpos] = hal[i];
+                            nxt[i] = ldo(W + (i * fso + nb), vo);
+                            hal[i] = ldo(W + (i * fso + nb), ho);
+                        }
+                        JFA_SCHED_BARRIER();
+                    });
+            }
+            slot = slot == NW - 2 ? 0 : slot + 1;
+            double rhs[5];
+#pragma unroll
+            for (int i = 0; i < 5; ++i) {
+                rhs[i] = (rr[i] + G.one_dx[A] * (Fp[i] - Fn[i])) + dz[i];  // space_solver.py:314
+                Fp[i] = Fn[i];
+            }
+            if (vcell) {
+                if (args.mode == 0) {
+#pragma unroll
+                    for (int i = 0; i < 5; ++i)
+                        args.rhs_out[i * ncell + rr0 + (roff / (uint32_t)sizeof(double))] = static_cast<T>(rhs[i]);
+                } else {
+                    double u[5], wn[5];
+#pragma unroll
+                    for (int i = 0; i < 5; ++i) {
+                        const double x = args.stage > 0 ? c0 * ui[i] + c1 * un[i] : ui[i];  // RK3.py:49-50
+                        u[i] = x + ts * rhs[i];                                             // time_integrator.py:57
+                    }
+                    prim_from_cons(u, prm, wn);
+#pragma unroll
+                    for (int i = 0; i < 5; ++i) {
+                        sto(args.Wout + (i * fso + rb), vo, wn[i]);
+                        sto(args.Uout + (i * fso + rb), vo, u[i]);
+                    }
+                    double uh[5];
+                    cons_from_prim(wn, prm, uh);
+                    int c[3];
+                    c[A] = a;
+                    c[O] = io;
+                    c[IN] = f;
+                    halo_scatter(args.Wout, args.Uout, G, args.bc, c, bl + rb, wn, uh, prm);
+                    if (args.cfl_part) vmax = nan_max(vmax, wave_sum(wn, G.active, prm.gamma));
+                }
+            }
+        }
+    }
+    if (args.cfl_part) block_max_part(args.cfl_part, vmax, blockIdx.x);
+}
+
 // dt from the per-block partials (time_step_size.py:103-135,154-155): dx_min / (max sum(|u|+c) + eps),
 // and with dissipative fluxes the minimum with 3/14 dx_min^2 / (max mu/rho + eps) (viscous) and
 // 0.1 dx_min^2 / (max kappa/(rho cp) + eps) (heat), times CFL.  part holds 1 or 3 arrays of n.
@@ -415,6 +676,29 @@ static inline int march_chunk(int nA, int64_t layer, int64_t slots, int64_t simd
     return best_L;
 }
 
+// Cut and chunk length of FINAL: L cells take 2 L + 1 faces, one more with aligned rows (the upper
+// faces).  can_pack: packs_rows of the row with its halo cells.  max_blocks: the CFL partials that
+// the workspace holds; false if no plan keeps to it.
+static inline bool final_plan(int nA, int nO, int N, bool can_pack, int64_t slots, int64_t simds, int64_t max_blocks,
+                              FinalPlan& p) {
+    const int64_t aligned = (int64_t)nO * ((N + 63) / 64);
+    const int64_t packed = ((int64_t)nO * (N + 6) + kPackStep - 1) / kPackStep;
+    double best = 1e300;
+    for (int pk = 0; pk < (can_pack ? 2 : 1); ++pk) {
+        const int64_t layer = pk ? packed : aligned;
+        for (int L = 1; L <= 64; ++L) {
+            const int64_t waves = layer * ((nA + L - 1) / L);
+            const double cost = rounds_time(waves, slots, simds) * (2 * L + (pk ? 1 : 2));
+            if ((waves + 3) / 4 <= max_blocks && waves < (int64_t)1 << 31 && cost < best * 0.999) {
+                best = cost;
+                p = {pk, L, (int)layer, (int)waves};
+            }
+            if (L >= nA) break;
+        }
+    }
+    return best < 1e300;
+}
+
 static inline int64_t device_cus() {
     static int num_cu = 0;
     if (num_cu == 0) {
@@ -434,19 +718,29 @@ static inline int64_t device_wave_slots(const void* kernel, int block) {
     return device_cus() * blocks * ((block + 63) / 64);
 }
 
-template <class T, int A, int IN, int VAR, int STENCIL, int RIEMANN, bool DISS, bool FLIM>
+template <class T, int A, int IN, int VAR, int STENCIL, int RIEMANN, bool DISS, bool FLIM, bool COMMON = false>
 static void launch_march(const void* W, const void* U, const Geo& G, const Params& prm, int accumulate, double* R,
                          hipStream_t st) {
     constexpr int O = 3 - A - IN;
     static int64_t slots = 0;
     if (slots == 0)
-        slots = device_wave_slots((const void*)march_kernel<T, A, IN, VAR, STENCIL, RIEMANN, DISS, FLIM>, kMarchBlock);
+        slots = device_wave_slots((const void*)march_kernel<T, A, IN, VAR, STENCIL, RIEMANN, DISS, FLIM, COMMON>, kMarchBlock);
     const int rowlen = packs_rows<T>(G, O, G.n[IN]) ? G.n[IN] : (G.n[IN] + 63) / 64 * 64;
     const int64_t cols = (int64_t)rowlen * G.n[O];
     const int L = march_chunk(G.n[A], (cols + 63) / 64, slots, 4 * device_cus());
     dim3 grid((unsigned)((cols + kMarchBlock - 1) / kMarchBlock), (unsigned)((G.n[A] + L - 1) / L));
-    hipLaunchKernelGGL((march_kernel<T, A, IN, VAR, STENCIL, RIEMANN, DISS, FLIM>), grid, dim3(kMarchBlock), 0, st,
+    hipLaunchKernelGGL((march_kernel<T, A, IN, VAR, STENCIL, RIEMANN, DISS, FLIM, COMMON>), grid, dim3(kMarchBlock), 0, st,
                        static_cast<const T*>(W), static_cast<const T*>(U), G, prm, L, rowlen, accumulate, R);
+}
+
+// Launches FINAL and returns its number of blocks.
+template <class T, int A, int IN, int VAR, int STENCIL, int RIEMANN>
+static int64_t launch_final(const void* W, const void* U, const Geo& G, const Params& prm, const InnerArgs<T>& a,
+                            const FinalPlan& plan, hipStream_t st) {
+    dim3 grid((unsigned)((plan.waves + 3) / 4));
+    hipLaunchKernelGGL((final_kernel<T, A, IN, VAR, STENCIL, RIEMANN>), grid, dim3(kInnerBlock), 0, st,
+                       static_cast<const T*>(W), static_cast<const T*>(U), G, prm, plan, a);
+    return grid.x;
 }
 
 template <class T, int IN, int VAR, int STENCIL, int RIEMANN, bool DISS, bool FLIM>
@@ -459,13 +753,40 @@ static int64_t launch_inner(const void* W, const void* U, const Geo& G, const Pa
 }
 
 // All sweeps of one stage (or of one RHS evaluation) for fixed scheme templates: a MARCH
-// kernel per active axis below IN, then the INNER kernel.  Returns the number of blocks of the
-// INNER launch (its CFL partials per quantity).
+// kernel per active axis below IN, then the INNER kernel, or FINAL in place of the last two.  Returns
+// the number of blocks of the last launch (its CFL partials per quantity).
 template <class T, int VAR, int STENCIL, int RIEMANN, bool DISS, bool FLIM>
 static int64_t sweeps(const void* W, const void* U, const Geo& G, const Params& prm, double* R, InnerArgs<T> ia,
                       hipStream_t st) {
     const int IN = innermost_axis(G);
     int acc = 0;
+    if constexpr (kFinal<VAR, STENCIL, RIEMANN, DISS, FLIM>) {
+        // The kernels of the common options hold them as constants; the others (the frozen state and
+        // signal speed switches and the face-state limiter cost scalar registers, whose spills cost
+        // FINAL 7 % and the x sweep 8 %) keep MARCH + INNER.  1-D grids have no axis to walk along.
+        const bool common = !prm.limiter && (VAR == JFA_PRIMITIVE || prm.frozen == JFA_FROZEN_ARITHMETIC) &&
+                            (RIEMANN == JFA_RUSANOV || prm.signal_speed == JFA_SS_EINFELDT);
+        if (common && IN > 0) {
+            const int A = IN == 1 || !G.active[1] ? 0 : 1;
+            FinalPlan plan;
+            static int64_t slots = 0;  // the (A, IN) variants hold the same registers and LDS
+            if (slots == 0)
+                slots = device_wave_slots((const void*)final_kernel<T, 1, 2, VAR, STENCIL, RIEMANN>, kInnerBlock);
+            const int O = 3 - A - IN;
+            if (final_plan(G.n[A], G.n[O], G.n[IN], packs_rows<T>(G, O, G.n[IN] + 6), slots, 4 * device_cus(),
+                           3 * inner_blocks(G), plan)) {
+                if (A == 1 && G.active[0]) {
+                    launch_march<T, 0, 2, VAR, STENCIL, RIEMANN, false, false, true>(W, U, G, prm, 0, R, st);
+                    acc = 1;
+                }
+                ia.R = R;
+                ia.accumulate = acc;
+                if (IN == 1) return launch_final<T, 0, 1, VAR, STENCIL, RIEMANN>(W, U, G, prm, ia, plan, st);
+                if (A == 0) return launch_final<T, 0, 2, VAR, STENCIL, RIEMANN>(W, U, G, prm, ia, plan, st);
+                return launch_final<T, 1, 2, VAR, STENCIL, RIEMANN>(W, U, G, prm, ia, plan, st);
+            }
+        }
+    }
     for (int A = 0; A < IN; ++A) {
         if (!G.active[A]) continue;
         if (A == 0 && IN == 1) launch_march<T, 0, 1, VAR, STENCIL, RIEMANN, DISS, FLIM>(W, U, G, prm, acc, R, st);
