@@ -8,7 +8,8 @@
 // for lane 63, from the extra upper face precomputed for the whole chunk (lane k holds the
 // extra face of plane x0+k).  The stage is then finished in registers: rhs = (0 + rhs_x) +
 // rhs_y (space_solver.py:266,314), RK3 blend/update, W = prim(U), stores, halo scatter,
-// CFL partial.  No scratch RHS, no LDS, no cross-wave synchronisation.
+// CFL partial.  No scratch RHS, no cross-wave synchronisation.  batch2d_walk_kernel keeps the wave's
+// rows in LDS (the common schemes), batch2d_stage_kernel reloads each face's window (the others).
 //
 // The grid holds one wavefront per item of every case; the hardware hands blocks to compute
 // units as they free up, which balances small and large cases without a software work queue
@@ -17,6 +18,7 @@
 #pragma once
 
 #include "jfa_common.h"
+#include "jfa_walk.h"
 
 namespace jfa {
 
@@ -108,6 +110,15 @@ __device__ __forceinline__ Geo geo_of(const Case2D& cs) {
     G.active[1] = 1;
     G.active[2] = 0;
     return G;
+}
+
+__device__ __forceinline__ BC6 boundaries_of(const Case2D& cs) {
+    BC6 bc;
+#pragma unroll
+    for (int f = 0; f < 4; ++f) bc.t[f] = cs.bc[f];
+    bc.t[4] = JFA_BC_PERIODIC;
+    bc.t[5] = JFA_BC_PERIODIC;
+    return bc;
 }
 
 // Flux of one face along AXIS (stride st): window cells -3..2 relative to the cell right of
@@ -251,13 +262,7 @@ __device__ __forceinline__ void run_item(const BatchArgs<T>& a, const Params& pr
             const int64_t bcell = rb + (int64_t)(yc + cs.nh);
             double uh[5];
             cons_from_prim(w, prm, uh);
-            BC6 bc;
-            bc.t[0] = cs.bc[0];
-            bc.t[1] = cs.bc[1];
-            bc.t[2] = cs.bc[2];
-            bc.t[3] = cs.bc[3];
-            bc.t[4] = JFA_BC_PERIODIC;
-            bc.t[5] = JFA_BC_PERIODIC;
+            const BC6 bc = boundaries_of(cs);
             const int c3[3] = {x, y, 0};
             halo_scatter(Wo, Uo, G, bc, c3, bcell, w, uh, prm);
             if (a.part) vmax = nan_max(vmax, wave_sum(w, G.active, prm.gamma));
@@ -281,6 +286,41 @@ void batch2d_stage_kernel(BatchArgs<T> a, Params prm) {
     BatchArgs<T> aa = a;
     if (a.part) aa.part = a.part + idx;
     run_item<T, VAR, STENCIL, RIEMANN, FLIM>(aa, prm, it);
+}
+
+// The common schemes (kFinal): the item's rows in LDS, every cell loaded once per plane, and the common
+// options as constants, as in the FINAL kernel (walk_rows).  Bound: FP64 issue at 226 VGPRs (two waves
+// per SIMD).  batch2d_stage_kernel fits three waves, but loads every window through L1 and spills
+// scalar registers into vector lanes: 64 cases of 128 .. 512 cells a side, CHAR-PRIMITIVE WENO5-JS
+// HLLC FP64, us per step: 1439 with it, 1076 with this kernel.
+template <class T, int VAR, int STENCIL, int RIEMANN>
+__global__ __launch_bounds__(kBatchBlock) JFA_WAVES_PER_EU(2) void batch2d_walk_kernel(BatchArgs<T> a, Params prm_) {
+    __shared__ WalkRows<STENCIL> rows[kBatchBlock / 64];
+    __shared__ double top[kBatchBlock / 64][5][64];
+    const unsigned idx = blockIdx.x * (kBatchBlock / 64) + (threadIdx.x >> 6);  // one item per wavefront
+    if (idx >= (unsigned)a.nitems) return;  // whole wavefronts only; no barriers follow
+    const Item2D it = load_item(a.items + idx);
+    const Case2D cs = load_case(a.cases + it.c);
+    const int lane = threadIdx.x & 63;
+    InnerArgs<T> args = {};
+    args.mode = 1;
+    args.Uin = a.Uin + cs.off;
+    args.Un = a.Un + cs.off;
+    args.Wout = a.Wout + cs.off;
+    args.Uout = a.Uout + cs.off;
+    args.bc = boundaries_of(cs);
+    args.stage = a.stage;
+    args.dt_host = uni(a.dt[it.c]);
+    args.cfl_part = a.part;
+    const int y = it.y0 + lane;
+    double vmax = walk_rows<T, 0, 1, VAR, STENCIL, RIEMANN>(a.Win + cs.off, a.Uin + cs.off, geo_of(cs),
+                                                            common_options(prm_), args, false, 0, 0, it.y0, y,
+                                                            y < cs.n1, it.x0, it.x1, rows[threadIdx.x >> 6],
+                                                            top[threadIdx.x >> 6]);
+    if (a.part) {
+        for (int o = 32; o > 0; o >>= 1) vmax = nan_max(vmax, __shfl_xor(vmax, o, 64));
+        if (lane == 0) a.part[idx] = vmax;
+    }
 }
 
 // WAVESPEED maxima of every case (max over its interior of |u| + c and |v| + c) into
@@ -353,6 +393,13 @@ template <class T, int VAR, int STENCIL, int RIEMANN>
 static void launch_batch(const BatchArgs<T>& a, const Params& prm, hipStream_t st) {
     const int waves_per_block = kBatchBlock / 64;
     const int blocks = (a.nitems + waves_per_block - 1) / waves_per_block;
+    if constexpr (kFinal<VAR, STENCIL, RIEMANN, false, false>) {  // the schemes of FINAL, at any size
+        if (!prm.flux_limiter && common_scheme<VAR, RIEMANN>(prm)) {
+            hipLaunchKernelGGL((batch2d_walk_kernel<T, VAR, STENCIL, RIEMANN>), dim3(blocks), dim3(kBatchBlock), 0, st,
+                               a, prm);
+            return;
+        }
+    }
     // the positivity flux limiter is a compile-time variant, so the plain kernel keeps its registers
     if (prm.flux_limiter)
         hipLaunchKernelGGL((batch2d_stage_kernel<T, VAR, STENCIL, RIEMANN, true>), dim3(blocks), dim3(kBatchBlock), 0,
