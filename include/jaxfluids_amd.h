@@ -329,9 +329,12 @@ int jfa_rk3_stage_fused_noalloc(const void* W_in, const void* U_in, const void* 
  *   lam_n  += c1 lam_out                                                  (stages 1, 2)
  * on interior cells; halos of lam_* are neither read nor written.  lam_in, lam_n and lam_out
  * must be distinct.  workspace: >= jfa_stage_vjp_workspace_bytes(grid, scheme) bytes (the face-halo
- * cotangents, plus 9 doubles per interior cell with a transport). */
+ * cotangents, plus 9 doubles per interior cell with a transport and, for PRIMITIVE reconstruction with
+ * a WENO5 stencil, 10 doubles per face of the axis with the most; a null scheme gives enough for any
+ * scheme without a transport). */
 size_t jfa_stage_vjp_workspace_bytes(const jfa_grid* grid, const jfa_scheme* scheme);
-/* Tuning of jfa_rk3_stage_vjp (process-wide): an axis other than the innermost is swept by the
+/* Tuning of jfa_rk3_stage_vjp (process-wide) for the schemes swept in one pass (all but PRIMITIVE
+ * reconstruction with a WENO5 stencil): an axis other than the innermost is swept by the
  * marching transpose kernel (coalesced columns, chunks of 16 cells) when that launch has at least
  * `waves` wavefronts, else by the lane-parallel one (one face per lane, strided loads).  Default
  * 2048; 0 forces marching, a huge value lane-parallel sweeps.  No reference counterpart (the

@@ -9,7 +9,8 @@
 // where halo^T sends the cotangent of every face-halo cell back to the interior cell the halo
 // fill copied it from (with the symmetric-wall sign flip).
 //
-// Kernels mirror the forward sweeps, transposed:
+// Kernels mirror the forward sweeps, transposed (PRIMITIVE reconstruction with a WENO5 stencil goes
+// face by face and cell by cell instead: adj_face_kernel, adj_cell_march_kernel, adj_cell_lane_kernel):
 // * adj_march_kernel (every active axis but the innermost): lanes along the innermost axis,
 //   each thread walks the faces of a column and accumulates window cotangents in a 6-cell
 //   register window; each chunk owns a range of cells and evaluates every face that touches
@@ -24,6 +25,8 @@
 // Face states are recomputed with the forward's own face_states, so branch choices (the sign
 // of S*, the min/max of the wave-speed estimates) are those of the forward evaluation.
 #pragma once
+
+#include <algorithm>
 
 #include "jfa_common.h"
 #include "jfa_dissipative.h"
@@ -49,7 +52,7 @@ __device__ __forceinline__ void weno5_vjp(double a, double b, double c, double d
     double al0, al1, al2, da0, da1, da2;  // alpha_k and d alpha_k / d beta_k
     double r0 = 0.0, r1 = 0.0, r2 = 0.0, tau = 0.0;
     if constexpr (STENCIL == JFA_WENO5_JS) {
-        const double q0 = 1.0 / (b0 * b0 + eps), q1 = 1.0 / (b1 * b1 + eps), q2 = 1.0 / (b2 * b2 + eps);
+        const double q0 = rcp(b0 * b0 + eps), q1 = rcp(b1 * b1 + eps), q2 = rcp(b2 * b2 + eps);
         al0 = d0 * q0;
         al1 = d1 * q1;
         al2 = d2 * q2;
@@ -58,9 +61,9 @@ __device__ __forceinline__ void weno5_vjp(double a, double b, double c, double d
         da2 = -2.0 * b2 * al2 * q2;
     } else {
         tau = fabs(b0 - b2);
-        r0 = 1.0 / (b0 + eps);
-        r1 = 1.0 / (b1 + eps);
-        r2 = 1.0 / (b2 + eps);
+        r0 = rcp(b0 + eps);
+        r1 = rcp(b1 + eps);
+        r2 = rcp(b2 + eps);
         al0 = d0 * (1.0 + tau * r0);
         al1 = d1 * (1.0 + tau * r1);
         al2 = d2 * (1.0 + tau * r2);
@@ -68,7 +71,7 @@ __device__ __forceinline__ void weno5_vjp(double a, double b, double c, double d
         da1 = -d1 * tau * r1 * r1;
         da2 = -d2 * tau * r2 * r2;
     }
-    const double iS = 1.0 / (al0 + al1 + al2);
+    const double iS = rcp(al0 + al1 + al2);
     const double w0 = al0 * iS, w1 = al1 * iS, w2 = al2 * iS;
     const double v = w0 * p0 + w1 * p1 + w2 * p2;
     // omega_k = alpha_k / S:  abar_k = vbar (p_k - v) / S
@@ -100,6 +103,75 @@ __device__ __forceinline__ void weno5_vjp(double a, double b, double c, double d
     ge += t2 + u2;
 }
 
+// Both states of a cell (weno5_cell: hi, the left state of the face above, from cells a..e around c;
+// lo, the right state of the face below, the mirrored stencil): out = vh d hi / d(a..e) + vl d lo / d(a..e).
+// The two states share the indicators and weights e_k, so their cotangents meet in e_k before they
+// go to q_k, the slopes and the cells.  With q_k the indicators of weno5_weights and
+// T_k = ebar_k prod_{j != k} q_j:  sum_k ebar_k e_k = 0 (hi and lo are homogeneous of degree zero in
+// e), which gives qbar_k = -tau T_k / q_k (+- sign(q_0 - q_2) sum T for k = 0, 2) for WENO-Z and
+// bbar_k = -2 b_k T_k / q_k for WENO-JS without cancelling terms.
+template <int STENCIL>
+__device__ __forceinline__ void weno5_cell_vjp(double a, double b, double c, double d, double e, double eps_z,
+                                               double eps_js, double vh, double vl, double out[5]) {
+    const double d0 = b - a, d1 = c - b, d2 = d - c, d3 = e - d;
+    const double D0 = d1 - d0, D1 = d2 - d1, D2 = d3 - d2;
+    const double S0 = fma(3.0, d1, -d0), S1 = d1 + d2, S2 = fma(-3.0, d2, d3);
+    const double b0 = fma(S0, S0, weno5_sq<STENCIL>(D0, eps_z)), b1 = fma(S1, S1, weno5_sq<STENCIL>(D1, eps_z)),
+                 b2 = fma(S2, S2, weno5_sq<STENCIL>(D2, eps_z));
+    double q0 = b0, q1 = b1, q2 = b2, tau = 0.0;
+    if constexpr (STENCIL == JFA_WENO5_JS) {
+        q0 = fma(b0, b0, eps_js);
+        q1 = fma(b1, b1, eps_js);
+        q2 = fma(b2, b2, eps_js);
+    } else {
+        tau = fabs(b0 - b2);
+    }
+    const double p12 = q1 * q2, p02 = q0 * q2, p01 = q0 * q1;
+    const double P = p01 * q2;
+    const double rP = rcp(P);
+    double e0 = p12, e1 = p02, e2 = p01;
+    if constexpr (STENCIL == JFA_WENO5_Z) {
+        e0 = fma(tau, p12, P);
+        e1 = fma(tau, p02, P);
+        e2 = fma(tau, p01, P);
+    }
+    // hi = c + N_h / M_h, lo = c + N_l / M_l (weno5_state)
+    const double gh0 = fma(5.0 / 6.0, d1, (-1.0 / 3.0) * d0), gh1 = fma(2.0, d2, d1), gh2 = fma(-0.5, d3, 2.0 * d2);
+    const double gl0 = fma(-5.0 / 6.0, d2, (1.0 / 3.0) * d3), gl1 = -fma(2.0, d1, d2), gl2 = fma(0.5, d0, -2.0 * d1);
+    const double rh = rcp(fma(3.0, e2, fma(6.0, e1, e0))), rl = rcp(fma(3.0, e0, fma(6.0, e1, e2)));
+    const double xh = fma(e2, gh2, fma(e1, gh1, e0 * gh0)) * rh, xl = fma(e0, gl2, fma(e1, gl1, e2 * gl0)) * rl;
+    const double nh = vh * rh, nl = vl * rl;  // cotangents of N_h, N_l; those of M are -n x
+    const double eb0 = fma(nh, gh0 - xh, nl * (gl2 - 3.0 * xl));
+    const double eb1 = fma(nh, gh1 - 6.0 * xh, nl * (gl1 - 6.0 * xl));
+    const double eb2 = fma(nh, gh2 - 3.0 * xh, nl * (gl0 - xl));
+    const double T0 = eb0 * p12, T1 = eb1 * p02, T2 = eb2 * p01;
+    const double t0 = T0 * (p12 * rP), t1 = T1 * (p02 * rP), t2 = T2 * (p01 * rP);  // T_k / q_k
+    double g0, g1, g2;  // cotangents of 4 beta_k
+    if constexpr (STENCIL == JFA_WENO5_JS) {
+        g0 = -2.0 * b0 * t0;
+        g1 = -2.0 * b1 * t1;
+        g2 = -2.0 * b2 * t2;
+    } else {
+        const double st = T0 + T1 + T2;
+        const double s = b0 > b2 ? st : (b0 < b2 ? -st : 0.0);
+        g0 = fma(-tau, t0, s);
+        g1 = -tau * t1;
+        g2 = fma(-tau, t2, -s);
+    }
+    const double Db0 = (2.0 * kQ) * D0 * g0, Db1 = (2.0 * kQ) * D1 * g1, Db2 = (2.0 * kQ) * D2 * g2;
+    const double Sb0 = 2.0 * S0 * g0, Sb1 = 2.0 * S1 * g1, Sb2 = 2.0 * S2 * g2;
+    const double h0 = nh * e0, h1 = nh * e1, h2 = nh * e2, l0 = nl * e2, l1 = nl * e1, l2 = nl * e0;
+    const double db0 = fma(-1.0 / 3.0, h0, 0.5 * l2) - Db0 - Sb0;
+    const double db1 = fma(5.0 / 6.0, h0, h1) - 2.0 * (l1 + l2) + (Db0 - Db1) + fma(3.0, Sb0, Sb1);
+    const double db2 = 2.0 * (h1 + h2) - fma(5.0 / 6.0, l0, l1) + (Db1 - Db2) + fma(-3.0, Sb2, Sb1);
+    const double db3 = fma(-0.5, h2, (1.0 / 3.0) * l0) + Db2 + Sb2;
+    out[0] = -db0;
+    out[1] = db0 - db1;
+    out[2] = (vh + vl) + (db1 - db2);
+    out[3] = db2 - db3;
+    out[4] = db3;
+}
+
 // ------------------------------------------------------------------ pointwise VJPs
 // U = cons(W) (equation_manager.py:93-101): adds (dU/dW)^T gU to gW.
 __device__ __forceinline__ void cons_vjp(const double W[5], const double gU[5], const Params& prm, double gW[5]) {
@@ -112,7 +184,7 @@ __device__ __forceinline__ void cons_vjp(const double W[5], const double gU[5], 
 
 // W = prim(U) (equation_manager.py:164-171): returns (dW/dU)^T gW, written with W.
 __device__ __forceinline__ void prim_vjp(const double W[5], const double gW[5], const Params& prm, double gU[5]) {
-    const double ir = 1.0 / W[0];
+    const double ir = rcp(W[0]);
     const double q2 = W[1] * W[1] + W[2] * W[2] + W[3] * W[3];
     gU[0] = gW[0] - (W[1] * gW[1] + W[2] * gW[2] + W[3] * gW[3]) * ir + prm.gm1 * 0.5 * q2 * gW[4];
 #pragma unroll
@@ -137,8 +209,9 @@ __device__ __forceinline__ void physical_flux_vjp(const double W[5], const doubl
 // c = sqrt(gamma p / rho) (ideal_gas.py:69-71)
 __device__ __forceinline__ void sound_speed_vjp(double c, double rho, double gamma, double gc, double& grho,
                                                 double& gp) {
-    gp += gc * gamma / (2.0 * c * rho);
-    grho -= gc * c / (2.0 * rho);
+    const double h = 0.5 * gc * rcp(rho);
+    gp += fdiv(h * gamma, c);
+    grho -= h * c;
 }
 
 // Shares of a min / max cotangent g for its operands x, y: all of it to the one the forward
@@ -242,14 +315,14 @@ __device__ __forceinline__ void signal_speeds_vjp(int kind, double uL, double uR
             gaR += g2;
         } break;
         default: {  // EINFELDT
-            const double sL = sqrt(rL), sR = sqrt(rR);
-            const double od = 1.0 / (sL + sR);
+            const double sL = fsqrt(rL), sR = fsqrt(rR);
+            const double od = rcp(sL + sR);
             const double eta2 = 0.5 * sL * sR * od * od;
             const double t2 = sL * uL + sR * uR;
             const double ub = t2 * od;
             const double du = uR - uL;
             const double t1 = sL * aL * aL + sR * aR * aR;
-            const double db = sqrt(t1 * od + eta2 * du * du);
+            const double db = fsqrt(t1 * od + eta2 * du * du);
             double gub = 0.0, gdb = 0.0, g1 = 0.0, g2 = 0.0;
             minmax_vjp(true, ub - db, uL - aL, gSL, g1, g2);
             gub += g1;
@@ -262,7 +335,7 @@ __device__ __forceinline__ void signal_speeds_vjp(int kind, double uL, double uR
             gdb += g1;
             guR += g2;
             gaR += g2;
-            const double gQ = db > 0.0 ? gdb / (2.0 * db) : 0.0;
+            const double gQ = db > 0.0 ? fdiv(0.5 * gdb, db) : 0.0;
             const double gt1 = gQ * od;
             double god = gQ * t1;
             const double geta2 = gQ * du * du;
@@ -284,8 +357,8 @@ __device__ __forceinline__ void signal_speeds_vjp(int kind, double uL, double uR
             const double gsum = -god * od * od;
             gsL += gsum;
             gsR += gsum;
-            grL += gsL / (2.0 * sL);
-            grR += gsR / (2.0 * sR);
+            grL += fdiv(0.5 * gsL, sL);
+            grR += fdiv(0.5 * gsR, sR);
         } break;
     }
 }
@@ -300,7 +373,7 @@ __device__ __forceinline__ void hllc_state_vjp(const double W[5], const double U
     constexpr int v = Ax<AXIS>::v, m0 = Ax<AXIS>::m0, m1 = Ax<AXIS>::m1;
     const double u = W[v];
     const double d = SK - u;
-    const double inv = 1.0 / (SK - Ss);
+    const double inv = rcp(SK - Ss);
     const double rd = W[0] * d;
     const double pre = rd * inv;
     const double A = Ss - u;
@@ -362,13 +435,13 @@ __device__ __forceinline__ void hllc_vjp(const double WL[5], const double WR[5],
                                          double gWR[5]) {
     constexpr int v = Ax<AXIS>::v;
     const double g = prm.gamma;
-    const double cL = sqrt(g * WL[4] / WL[0]), cR = sqrt(g * WR[4] / WR[0]);
+    const double cL = fsqrt(fdiv(g * WL[4], WL[0])), cR = fsqrt(fdiv(g * WR[4], WR[0]));
     double SL, SR;
     signal_speeds(prm.signal_speed, WL[v], WR[v], cL, cR, WL[0], WR[0], WL[4], WR[4], g, SL, SR);
     const double aL = WL[0] * (SL - WL[v]), aR = WR[0] * (SR - WR[v]);
     const double num = (WR[4] - WL[4]) + (WL[v] * aL - WR[v] * aR);
     const double den = aL - aR;
-    const double Ss = num / den;
+    const double Ss = fdiv(num, den);
     double gUL[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, gUR[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     double gSL = 0.0, gSR = 0.0, gSs = 0.0;
     if (Ss >= 0.0) {
@@ -384,7 +457,7 @@ __device__ __forceinline__ void hllc_vjp(const double WL[5], const double WR[5],
         hllc_star_vjp<AXIS, false>(WR, UR, SR, Ss, m, gWR, gUR, gSR, gSs);
     }
     // S* = num / den (signal_speeds.py:194-197)
-    const double gnum = gSs / den, gden = -gSs * Ss / den;
+    const double gnum = fdiv(gSs, den), gden = -gnum * Ss;
     gWR[4] += gnum;
     gWL[4] -= gnum;
     gWL[v] += gnum * aL;
@@ -413,7 +486,7 @@ __device__ __forceinline__ void hll_vjp(const double WL[5], const double WR[5], 
                                         double gWR[5]) {
     constexpr int v = Ax<AXIS>::v;
     const double g = prm.gamma;
-    const double cL = sqrt(g * WL[4] / WL[0]), cR = sqrt(g * WR[4] / WR[0]);
+    const double cL = fsqrt(fdiv(g * WL[4], WL[0])), cR = fsqrt(fdiv(g * WR[4], WR[0]));
     double SL, SR;
     signal_speeds(prm.signal_speed, WL[v], WR[v], cL, cR, WL[0], WR[0], WL[4], WR[4], g, SL, SR);
     const double sl = fmin(SL, 0.0), sr = fmax(SR, 0.0);
@@ -462,13 +535,13 @@ __device__ __forceinline__ void hllc_lm_vjp(const double WL[5], const double WR[
                                             double gWL[5], double gWR[5]) {
     constexpr int v = Ax<AXIS>::v;
     const double g = prm.gamma;
-    const double cL = sqrt(g * WL[4] / WL[0]), cR = sqrt(g * WR[4] / WR[0]);
+    const double cL = fsqrt(fdiv(g * WL[4], WL[0])), cR = fsqrt(fdiv(g * WR[4], WR[0]));
     double SL, SR;
     signal_speeds(prm.signal_speed, WL[v], WR[v], cL, cR, WL[0], WR[0], WL[4], WR[4], g, SL, SR);
     const double aL = WL[0] * (SL - WL[v]), aR = WR[0] * (SR - WR[v]);
     const double num = (WR[4] - WL[4]) + (WL[v] * aL - WR[v] * aR);
     const double den = aL - aR;
-    const double Ss = num / den;
+    const double Ss = fdiv(num, den);
     double usL[5], usR[5];
     hllc_star_state<AXIS>(WL, UL, SL, Ss, usL);
     hllc_star_state<AXIS>(WR, UR, SR, Ss, usR);
@@ -510,7 +583,7 @@ __device__ __forceinline__ void hllc_lm_vjp(const double WL[5], const double WR[
     hllc_state_vjp<AXIS>(WL, UL, SL, Ss, gusL, gWL, gUL, gSL, gSs);
     hllc_state_vjp<AXIS>(WR, UR, SR, Ss, gusR, gWR, gUR, gSR, gSs);
     // S* = num / den (signal_speeds.py:194-197)
-    const double gnum = gSs / den, gden = -gSs * Ss / den;
+    const double gnum = fdiv(gSs, den), gden = -gnum * Ss;
     gWR[4] += gnum;
     gWL[4] -= gnum;
     gWL[v] += gnum * aL;
@@ -541,7 +614,7 @@ __device__ __forceinline__ void ausmp_vjp(const double WL[5], const double WR[5]
     constexpr int v = Ax<AXIS>::v;
     constexpr double alpha = 3.0 / 16.0, beta = 1.0 / 8.0;
     const double g = prm.gamma;
-    const double cL = sqrt(g * WL[4] / WL[0]), cR = sqrt(g * WR[4] / WR[0]);
+    const double cL = fsqrt(fdiv(g * WL[4], WL[0])), cR = fsqrt(fdiv(g * WR[4], WR[0]));
     const double a = 0.5 * (cL + cR);
     const double Ml = WL[v] / a, Mr = WR[v] / a;
     const double ql = Ml * Ml - 1.0, qr = Mr * Mr - 1.0;
@@ -595,7 +668,7 @@ __device__ __forceinline__ void rusanov_vjp(const double WL[5], const double WR[
                                             double gWL[5], double gWR[5]) {
     constexpr int v = Ax<AXIS>::v;
     const double g = prm.gamma;
-    const double cL = sqrt(g * WL[4] / WL[0]), cR = sqrt(g * WR[4] / WR[0]);
+    const double cL = fsqrt(fdiv(g * WL[4], WL[0])), cR = fsqrt(fdiv(g * WR[4], WR[0]));
     const double alpha = fmax(fabs(WL[v]) + cL, fabs(WR[v]) + cR);
     double gUL[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, gUR[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, half[5];
     double galpha = 0.0;
@@ -1626,6 +1699,139 @@ __global__ __launch_bounds__(kAdjBlock) void adj_march_kernel(const double* __re
     }
 }
 
+// ------------------------------------------------------------------ PRIMITIVE in two passes
+// PRIMITIVE reconstruction with the WENO5 stencils: every variable of a cell is reconstructed from
+// the cell's own five-cell stencil, so the face's work and the cells' separate.
+// * adj_face_kernel: one thread per face, its cotangents of W_L and W_R (10 doubles) into GF.
+// * adj_cell_march_kernel / adj_cell_lane_kernel: one variable per thread (grid dimension); centre
+//   cell c takes the cotangents of its two states (W_L of face c + 1, W_R of face c) through
+//   weno5_cell_vjp to the cells c - 2 .. c + 2.
+// Against the one-pass sweeps below: a face's states and Riemann reverse are evaluated once (a
+// marching chunk repeats 5 faces of 21), the WENO indicators once per cell (four times a face), and
+// the cell pass needs few registers.  The price is 80 bytes written and read per face, and the cell
+// pass is bound by them (3.6 of the 4.8 TB/s a copy reaches); the face pass is bound by FP64 issue.
+// 128^3, WENO5-Z HLLC, us per stage along x / y / z: 536 / 498 / 338 in one pass, 263 / 250 / 267 in two.
+template <int VAR, int STENCIL, int RIEMANN>
+constexpr bool kTwoPass = VAR == JFA_PRIMITIVE && (STENCIL == JFA_WENO5_JS || STENCIL == JFA_WENO5_Z) &&
+                          RIEMANN != kFluxSplit;
+
+template <int A, int STENCIL, int RIEMANN>
+__global__ __launch_bounds__(kAdjBlock) void adj_face_kernel(const double* __restrict__ W,
+                                                             const double* __restrict__ lam, Geo G, FaceIdx F,
+                                                             Params prm, double ts, double* __restrict__ GF) {
+    int f[3];
+    if (!flat_index(F.nface, F.fe[1], F.fe[2], f[0], f[1], f[2])) return;
+    const int64_t br = (int64_t)(f[0] + G.off[0]) * G.s[0] + (int64_t)(f[1] + G.off[1]) * G.s[1] + (f[2] + G.off[2]);
+    double mu[5], gl[5], gr[5], fz[FZ_N];
+    face_mu(lam, br, G.s[A], G.fs, f[A], G.n[A], ts * G.one_dx[A], mu);
+    face_state_vjp_at<A, STENCIL, RIEMANN, JFA_PRIMITIVE>(W, br, G.s[A], G.fs, mu, prm, gl, gr, fz);
+    const int64_t o = ((int64_t)f[0] * F.fe[1] + f[1]) * F.fe[2] + f[2];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        JFA_ACCESS(GF + i * F.nface + o, sizeof(double));
+        JFA_ACCESS(GF + (5 + i) * F.nface + o, sizeof(double));
+        GF[i * F.nface + o] = gl[i];
+        GF[(5 + i) * F.nface + o] = gr[i];
+    }
+}
+
+// Cell pass along A: lanes over the columns (buffer order of IN), chunk blockIdx.y owns the cells
+// [-3 + y L, -3 + (y + 1) L) of its columns and walks the centres that reach them, variable blockIdx.z.
+template <int A, int IN, int STENCIL>
+__global__ __launch_bounds__(kAdjBlock) void adj_cell_march_kernel(const double* __restrict__ W,
+                                                                   const double* __restrict__ GF, Geo G, FaceIdx F,
+                                                                   Params prm, int L, double* __restrict__ gW) {
+    constexpr int O = 3 - A - IN;
+    const int col = blockIdx.x * kAdjBlock + threadIdx.x;
+    const int io = col / G.n[IN], iin = col - io * G.n[IN];
+    if (io >= G.n[O]) return;  // no barriers in this kernel
+    const int i = blockIdx.z;
+    const int N = G.n[A];
+    const int o0 = -3 + (int)blockIdx.y * L, o1 = min(o0 + L, N + 3);
+    const int ca = max(o0 - 2, -1), cb = min(o1 + 1, N);
+    const int64_t sa = G.s[A];
+    const int64_t b0 = (int64_t)i * G.fs + (int64_t)(io + G.off[O]) * G.s[O] + (int64_t)(iin + G.off[IN]) * G.s[IN] +
+                       (int64_t)G.off[A] * sa;  // field i, cell 0 along A
+    const int64_t fsA = A == 0 ? (int64_t)F.fe[1] * F.fe[2] : (A == 1 ? (int64_t)F.fe[2] : 1);
+    const int64_t fsO = O == 0 ? (int64_t)F.fe[1] * F.fe[2] : (O == 1 ? (int64_t)F.fe[2] : 1);
+    const int64_t fsI = IN == 0 ? (int64_t)F.fe[1] * F.fe[2] : (IN == 1 ? (int64_t)F.fe[2] : 1);
+    const int64_t fl = i * F.nface + io * fsO + iin * fsI, fr = fl + 5 * F.nface;  // face 0 along A
+    double x[5], acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) x[k + 1] = ld(W, b0 + (int64_t)(ca - 2 + k) * sa);
+    auto put = [&](int cell, double v) {
+        if (cell >= o0 && cell < o1) {
+            double* p = gW + b0 + (int64_t)cell * sa;
+            JFA_ACCESS(p, sizeof(double));
+            *p += v;
+        }
+    };
+    for (int c = ca; c <= cb; ++c) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[k] = x[k + 1];
+        x[4] = ld(W, b0 + (int64_t)(c + 2) * sa);
+        const double vh = c < N ? ld(GF, fl + (c + 1) * fsA) : 0.0;
+        const double vl = c >= 0 ? ld(GF, fr + c * fsA) : 0.0;
+        double o[5];
+        weno5_cell_vjp<STENCIL>(x[0], x[1], x[2], x[3], x[4], prm.eps_z, prm.eps_js, vh, vl, o);
+#pragma unroll
+        for (int k = 0; k < 5; ++k) acc[k] += o[k];
+        put(c - 2, acc[0]);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) acc[k] = acc[k + 1];
+        acc[4] = 0.0;
+    }
+    if (cb == N) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) put(N - 1 + k, acc[k]);
+    }
+}
+
+// Cell pass along the innermost axis: one centre per lane, a cell gathers from the five centres
+// around it by wave shuffles; wave w of a row owns the cells -3 + 60 w + (0 .. 59), its lanes the
+// centres -5 + 60 w + (0 .. 63).  Variable blockIdx.y.
+template <int A, int STENCIL>
+__global__ __launch_bounds__(kAdjBlock) void adj_cell_lane_kernel(const double* __restrict__ W,
+                                                                  const double* __restrict__ GF, Geo G, FaceIdx F,
+                                                                  Params prm, int waves_per_row, int64_t nwaves,
+                                                                  double* __restrict__ gW) {
+    constexpr int P = A == 0 ? 1 : 0;
+    constexpr int Q = A == 2 ? 1 : 2;
+    const int64_t gwave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    const int lane = threadIdx.x & 63;
+    const bool vwave = gwave < nwaves;  // whole waves; shuffles below run in every lane of a wave
+    const int64_t row = vwave ? gwave / waves_per_row : 0;
+    const int w = vwave ? (int)(gwave - row * waves_per_row) : 0;
+    const int N = G.n[A], i = blockIdx.y;
+    const int cP = (int)(row / G.n[Q]);
+    const int cQ = (int)(row - (int64_t)cP * G.n[Q]);
+    const int64_t sa = G.s[A];
+    const int64_t b0 = (int64_t)i * G.fs + (int64_t)(cP + G.off[P]) * G.s[P] + (int64_t)(cQ + G.off[Q]) * G.s[Q] +
+                       (int64_t)G.off[A] * sa;
+    const int c = -5 + 60 * w + lane;
+    const bool centre = vwave && c >= -1 && c <= N;
+    double o[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    if (centre) {
+        const int64_t fsA = A == 0 ? (int64_t)F.fe[1] * F.fe[2] : (A == 1 ? (int64_t)F.fe[2] : 1);
+        const int64_t fsP = P == 0 ? (int64_t)F.fe[1] * F.fe[2] : (int64_t)F.fe[2];
+        const int64_t fsQ = Q == 1 ? (int64_t)F.fe[2] : 1;
+        const int64_t fl = i * F.nface + cP * fsP + cQ * fsQ, fr = fl + 5 * F.nface;
+        const int64_t bc = b0 + (int64_t)c * sa;
+        const double vh = c < N ? ld(GF, fl + (c + 1) * fsA) : 0.0;
+        const double vl = c >= 0 ? ld(GF, fr + c * fsA) : 0.0;
+        weno5_cell_vjp<STENCIL>(ld(W, bc - 2 * sa), ld(W, bc - sa), ld(W, bc), ld(W, bc + sa), ld(W, bc + 2 * sa),
+                                prm.eps_z, prm.eps_js, vh, vl, o);
+    }
+    const double s = o[2] + __shfl_up(o[3], 1u, 64) + __shfl_up(o[4], 2u, 64) + __shfl_down(o[1], 1u, 64) +
+                     __shfl_down(o[0], 2u, 64);
+    if (vwave && lane >= 2 && lane < 62 && c <= N + 2) {
+        double* p = gW + b0 + (int64_t)c * sa;
+        JFA_ACCESS(p, sizeof(double));
+        *p += s;
+    }
+}
+
+
 // Lane-parallel transpose sweep along axis A (stride s[A]; unit stride on the innermost axis).
 // Wave w of a row evaluates the faces F0 .. F0+63, F0 = -5 + 59 w (lane l: face F0 + l, zero
 // outside 0..N) and lanes 5..63 own the cells F0 + l - 3, i.e. [-3 + 59 w, -3 + 59 w + 59)
@@ -1974,49 +2180,97 @@ static inline int64_t march_waves(const Geo& G, int A, int IN) {
 // (strided loads along A, every face its own lane) is used for that axis instead.
 int64_t adjoint_march_min_waves();
 
-// Transpose sweeps of the convective flux along every active axis into gW.
+// Faces of the axis with the most, the face cotangents of one axis at a time (kTwoPass).
+static inline int64_t max_faces(const Geo& G) {
+    int64_t m = 0;
+    for (int a = 0; a < 3; ++a)
+        if (G.active[a]) m = std::max(m, face_extents(G, a).nface);
+    return m;
+}
+
+// The two passes along axis A.  Chunks of the marching cell pass: the longest of 64, 32, 16, 8 (4
+// centres more than cells each) that still fills the device four times over.
+template <int A, int IN, int STENCIL, int RIEMANN>
+static void launch_two_pass(const double* W, const double* lam, const Geo& G, const Params& prm, double ts, double* GF,
+                            double* gW, hipStream_t st) {
+    const FaceIdx F = face_extents(G, A);
+    hipLaunchKernelGGL((adj_face_kernel<A, STENCIL, RIEMANN>), flat_grid(F.nface), dim3(kAdjBlock), 0, st, W, lam, G, F,
+                       prm, ts, GF);
+    if constexpr (A == IN) {
+        constexpr int P = A == 0 ? 1 : 0, Q = A == 2 ? 1 : 2;
+        const int waves_per_row = (G.n[A] + 6 + 59) / 60;
+        const int64_t nwaves = (int64_t)waves_per_row * G.n[P] * G.n[Q];
+        const int64_t blocks = (nwaves + kAdjBlock / 64 - 1) / (kAdjBlock / 64);
+        hipLaunchKernelGGL((adj_cell_lane_kernel<A, STENCIL>), dim3((unsigned)blocks, 5), dim3(kAdjBlock), 0, st, W, GF,
+                           G, F, prm, waves_per_row, nwaves, gW);
+    } else {
+        constexpr int O = 3 - A - IN;
+        const int64_t cols = (int64_t)G.n[IN] * G.n[O], cells = G.n[A] + 6;
+        int L = 64;
+        while (L > 8 && 5 * ((cols + 63) / 64) * ((cells + L - 1) / L) < 16384) L /= 2;
+        hipLaunchKernelGGL((adj_cell_march_kernel<A, IN, STENCIL>),
+                           dim3((unsigned)((cols + kAdjBlock - 1) / kAdjBlock), (unsigned)((cells + L - 1) / L), 5),
+                           dim3(kAdjBlock), 0, st, W, GF, G, F, prm, L, gW);
+    }
+}
+
+// Transpose sweeps of the convective flux along every active axis into gW; GF: 10 doubles per face
+// of the axis with the most (kTwoPass schemes).
 template <int STENCIL, int RIEMANN, int VAR>
 static void adj_sweeps(const double* W, const double* lam, const Geo& G, const Params& prm, double ts, double* gW,
-                       hipStream_t st) {
+                       double* GF, hipStream_t st) {
     const int IN = innermost_axis(G);
-    const int64_t min_waves = adjoint_march_min_waves();
-    for (int A = 0; A < IN; ++A) {
-        if (!G.active[A]) continue;
-        if (march_waves(G, A, IN) < min_waves) {
-            if (A == 0) launch_adj_lanes<0, STENCIL, RIEMANN, VAR>(W, lam, G, prm, ts, gW, st);
-            else launch_adj_lanes<1, STENCIL, RIEMANN, VAR>(W, lam, G, prm, ts, gW, st);
-        } else if (A == 0 && IN == 1) {
-            launch_adj_march<0, 1, STENCIL, RIEMANN, VAR>(W, lam, G, prm, ts, gW, st);
-        } else if (A == 0) {
-            launch_adj_march<0, 2, STENCIL, RIEMANN, VAR>(W, lam, G, prm, ts, gW, st);
+    if constexpr (kTwoPass<VAR, STENCIL, RIEMANN>) {
+        if (IN == 0) {
+            launch_two_pass<0, 0, STENCIL, RIEMANN>(W, lam, G, prm, ts, GF, gW, st);
+        } else if (IN == 1) {
+            if (G.active[0]) launch_two_pass<0, 1, STENCIL, RIEMANN>(W, lam, G, prm, ts, GF, gW, st);
+            launch_two_pass<1, 1, STENCIL, RIEMANN>(W, lam, G, prm, ts, GF, gW, st);
         } else {
-            launch_adj_march<1, 2, STENCIL, RIEMANN, VAR>(W, lam, G, prm, ts, gW, st);
+            if (G.active[0]) launch_two_pass<0, 2, STENCIL, RIEMANN>(W, lam, G, prm, ts, GF, gW, st);
+            if (G.active[1]) launch_two_pass<1, 2, STENCIL, RIEMANN>(W, lam, G, prm, ts, GF, gW, st);
+            launch_two_pass<2, 2, STENCIL, RIEMANN>(W, lam, G, prm, ts, GF, gW, st);
         }
+    } else {
+        const int64_t min_waves = adjoint_march_min_waves();
+        for (int A = 0; A < IN; ++A) {
+            if (!G.active[A]) continue;
+            if (march_waves(G, A, IN) < min_waves) {
+                if (A == 0) launch_adj_lanes<0, STENCIL, RIEMANN, VAR>(W, lam, G, prm, ts, gW, st);
+                else launch_adj_lanes<1, STENCIL, RIEMANN, VAR>(W, lam, G, prm, ts, gW, st);
+            } else if (A == 0 && IN == 1) {
+                launch_adj_march<0, 1, STENCIL, RIEMANN, VAR>(W, lam, G, prm, ts, gW, st);
+            } else if (A == 0) {
+                launch_adj_march<0, 2, STENCIL, RIEMANN, VAR>(W, lam, G, prm, ts, gW, st);
+            } else {
+                launch_adj_march<1, 2, STENCIL, RIEMANN, VAR>(W, lam, G, prm, ts, gW, st);
+            }
+        }
+        if (IN == 0) launch_adj_lanes<0, STENCIL, RIEMANN, VAR>(W, lam, G, prm, ts, gW, st);
+        else if (IN == 1) launch_adj_lanes<1, STENCIL, RIEMANN, VAR>(W, lam, G, prm, ts, gW, st);
+        else launch_adj_lanes<2, STENCIL, RIEMANN, VAR>(W, lam, G, prm, ts, gW, st);
     }
-    if (IN == 0) launch_adj_lanes<0, STENCIL, RIEMANN, VAR>(W, lam, G, prm, ts, gW, st);
-    else if (IN == 1) launch_adj_lanes<1, STENCIL, RIEMANN, VAR>(W, lam, G, prm, ts, gW, st);
-    else launch_adj_lanes<2, STENCIL, RIEMANN, VAR>(W, lam, G, prm, ts, gW, st);
 }
 
 // adj_sweeps for a Riemann solver chosen at run time.
 template <int STENCIL, int VAR>
 inline void adj_sweeps_r(int riemann, const double* W, const double* lam, const Geo& G, const Params& prm, double ts,
-                         double* gW, hipStream_t st) {
+                         double* gW, double* GF, hipStream_t st) {
     if (riemann == JFA_FS_ROE || riemann == JFA_FS_CLLF || riemann == JFA_FS_LLF) {
         // the flux-splitting face flux reads the primitive window (the scheme's variable is unused)
-        if constexpr (VAR == JFA_PRIMITIVE) adj_sweeps<STENCIL, kFluxSplit, JFA_PRIMITIVE>(W, lam, G, prm, ts, gW, st);
+        if constexpr (VAR == JFA_PRIMITIVE) adj_sweeps<STENCIL, kFluxSplit, JFA_PRIMITIVE>(W, lam, G, prm, ts, gW, GF, st);
         return;
     }
-    if (riemann == JFA_HLLC) adj_sweeps<STENCIL, JFA_HLLC, VAR>(W, lam, G, prm, ts, gW, st);
-    else if (riemann == JFA_HLL) adj_sweeps<STENCIL, JFA_HLL, VAR>(W, lam, G, prm, ts, gW, st);
-    else if (riemann == JFA_HLLC_LM) adj_sweeps<STENCIL, JFA_HLLC_LM, VAR>(W, lam, G, prm, ts, gW, st);
-    else if (riemann == JFA_AUSMP) adj_sweeps<STENCIL, JFA_AUSMP, VAR>(W, lam, G, prm, ts, gW, st);
-    else adj_sweeps<STENCIL, JFA_RUSANOV, VAR>(W, lam, G, prm, ts, gW, st);
+    if (riemann == JFA_HLLC) adj_sweeps<STENCIL, JFA_HLLC, VAR>(W, lam, G, prm, ts, gW, GF, st);
+    else if (riemann == JFA_HLL) adj_sweeps<STENCIL, JFA_HLL, VAR>(W, lam, G, prm, ts, gW, GF, st);
+    else if (riemann == JFA_HLLC_LM) adj_sweeps<STENCIL, JFA_HLLC_LM, VAR>(W, lam, G, prm, ts, gW, GF, st);
+    else if (riemann == JFA_AUSMP) adj_sweeps<STENCIL, JFA_AUSMP, VAR>(W, lam, G, prm, ts, gW, GF, st);
+    else adj_sweeps<STENCIL, JFA_RUSANOV, VAR>(W, lam, G, prm, ts, gW, GF, st);
 }
 
 // The sweeps of the run-time-selected stencils (WENO1, WENO3-JS/-Z, TENO5, TENO5-A;
 // jfa_adjoint_ext.hip, a translation unit of its own).
 void adj_sweeps_ext(int var, int riemann, const double* W, const double* lam, const Geo& G, const Params& prm,
-                    double ts, double* gW, hipStream_t st);
+                    double ts, double* gW, double* GF, hipStream_t st);
 
 }  // namespace jfa

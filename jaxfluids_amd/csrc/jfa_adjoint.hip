@@ -23,6 +23,10 @@ int jfa_adjoint_set_march_min_waves(int64_t waves) {
 
 static size_t vjp_workspace_bytes(const Geo& G, const jfa_scheme* scheme) {
     size_t n = (size_t)(5 * G.fs);
+    // face cotangents of one axis (kTwoPass); without a scheme, enough for any
+    if (!scheme || (scheme->recon_var == JFA_PRIMITIVE && scheme->riemann < JFA_FS_ROE &&
+                    (scheme->stencil == JFA_WENO5_JS || scheme->stencil == JFA_WENO5_Z)))
+        n += (size_t)(10 * max_faces(G));
     if (scheme && scheme->transport && (scheme->transport->viscous || scheme->transport->heat))
         n += (size_t)9 * ((size_t)G.n[0] * G.n[1] * G.n[2]);  // X: transverse-derivative cotangent sums
     return n * sizeof(double);
@@ -78,33 +82,33 @@ int jfa_rk3_stage_vjp(const void* W_in, const void* lam_out, void* lam_in, void*
     hipStream_t st = (hipStream_t)stream;
     double* gW = static_cast<double*>(workspace);
     const int64_t nz = 5 * G.fs;
+    double* X = prm.dissip ? gW + nz : nullptr;  // written whole by the cell kernel: no clearing
+    double* GF = gW + nz + (prm.dissip ? 9 * (int64_t)G.n[0] * G.n[1] * G.n[2] : 0);
     const int64_t zb = (nz + kBlock - 1) / kBlock;
     hipLaunchKernelGGL(adj_zero_kernel<0>, dim3((unsigned)(zb < 4096 ? zb : 4096)), dim3(kBlock), 0, st, gW, nz);
     const double* W = static_cast<const double*>(W_in);
     const double* lam = static_cast<const double*>(lam_out);
     const int var = fsplit ? JFA_PRIMITIVE : scheme->recon_var;  // flux splitting: the primitive window
     if (ext) {
-        adj_sweeps_ext(var, scheme->riemann, W, lam, G, prm, m * dt, gW, st);
+        adj_sweeps_ext(var, scheme->riemann, W, lam, G, prm, m * dt, gW, GF, st);
     } else if (scheme->stencil == JFA_WENO5_JS) {
         if (var == JFA_CHAR_PRIMITIVE)
-            adj_sweeps_r<JFA_WENO5_JS, JFA_CHAR_PRIMITIVE>(scheme->riemann, W, lam, G, prm, m * dt, gW, st);
+            adj_sweeps_r<JFA_WENO5_JS, JFA_CHAR_PRIMITIVE>(scheme->riemann, W, lam, G, prm, m * dt, gW, GF, st);
         else if (var == JFA_CONSERVATIVE)
-            adj_sweeps_r<JFA_WENO5_JS, JFA_CONSERVATIVE>(scheme->riemann, W, lam, G, prm, m * dt, gW, st);
+            adj_sweeps_r<JFA_WENO5_JS, JFA_CONSERVATIVE>(scheme->riemann, W, lam, G, prm, m * dt, gW, GF, st);
         else if (var == JFA_CHAR_CONSERVATIVE)
-            adj_sweeps_r<JFA_WENO5_JS, JFA_CHAR_CONSERVATIVE>(scheme->riemann, W, lam, G, prm, m * dt, gW, st);
-        else adj_sweeps_r<JFA_WENO5_JS, JFA_PRIMITIVE>(scheme->riemann, W, lam, G, prm, m * dt, gW, st);
+            adj_sweeps_r<JFA_WENO5_JS, JFA_CHAR_CONSERVATIVE>(scheme->riemann, W, lam, G, prm, m * dt, gW, GF, st);
+        else adj_sweeps_r<JFA_WENO5_JS, JFA_PRIMITIVE>(scheme->riemann, W, lam, G, prm, m * dt, gW, GF, st);
     } else {
         if (var == JFA_CHAR_PRIMITIVE)
-            adj_sweeps_r<JFA_WENO5_Z, JFA_CHAR_PRIMITIVE>(scheme->riemann, W, lam, G, prm, m * dt, gW, st);
+            adj_sweeps_r<JFA_WENO5_Z, JFA_CHAR_PRIMITIVE>(scheme->riemann, W, lam, G, prm, m * dt, gW, GF, st);
         else if (var == JFA_CONSERVATIVE)
-            adj_sweeps_r<JFA_WENO5_Z, JFA_CONSERVATIVE>(scheme->riemann, W, lam, G, prm, m * dt, gW, st);
+            adj_sweeps_r<JFA_WENO5_Z, JFA_CONSERVATIVE>(scheme->riemann, W, lam, G, prm, m * dt, gW, GF, st);
         else if (var == JFA_CHAR_CONSERVATIVE)
-            adj_sweeps_r<JFA_WENO5_Z, JFA_CHAR_CONSERVATIVE>(scheme->riemann, W, lam, G, prm, m * dt, gW, st);
-        else adj_sweeps_r<JFA_WENO5_Z, JFA_PRIMITIVE>(scheme->riemann, W, lam, G, prm, m * dt, gW, st);
+            adj_sweeps_r<JFA_WENO5_Z, JFA_CHAR_CONSERVATIVE>(scheme->riemann, W, lam, G, prm, m * dt, gW, GF, st);
+        else adj_sweeps_r<JFA_WENO5_Z, JFA_PRIMITIVE>(scheme->riemann, W, lam, G, prm, m * dt, gW, GF, st);
     }
-    double* X = nullptr;
     if (prm.dissip) {
-        X = gW + nz;  // written whole by the cell kernel: no clearing
         hipLaunchKernelGGL(adj_dissip_cell_kernel<0>, flat_grid((int64_t)G.n[0] * G.n[1] * G.n[2]), dim3(kBlock), 0,
                            st, W, lam, G, prm, m * dt, gW, X);
     }

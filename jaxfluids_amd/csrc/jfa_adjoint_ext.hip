@@ -6,12 +6,12 @@
 namespace jfa {
 
 void adj_sweeps_ext(int var, int riemann, const double* W, const double* lam, const Geo& G, const Params& prm,
-                    double ts, double* gW, hipStream_t st) {
-    if (var == JFA_CHAR_PRIMITIVE) adj_sweeps_r<kStencilExt, JFA_CHAR_PRIMITIVE>(riemann, W, lam, G, prm, ts, gW, st);
-    else if (var == JFA_CONSERVATIVE) adj_sweeps_r<kStencilExt, JFA_CONSERVATIVE>(riemann, W, lam, G, prm, ts, gW, st);
+                    double ts, double* gW, double* GF, hipStream_t st) {
+    if (var == JFA_CHAR_PRIMITIVE) adj_sweeps_r<kStencilExt, JFA_CHAR_PRIMITIVE>(riemann, W, lam, G, prm, ts, gW, GF, st);
+    else if (var == JFA_CONSERVATIVE) adj_sweeps_r<kStencilExt, JFA_CONSERVATIVE>(riemann, W, lam, G, prm, ts, gW, GF, st);
     else if (var == JFA_CHAR_CONSERVATIVE)
-        adj_sweeps_r<kStencilExt, JFA_CHAR_CONSERVATIVE>(riemann, W, lam, G, prm, ts, gW, st);
-    else adj_sweeps_r<kStencilExt, JFA_PRIMITIVE>(riemann, W, lam, G, prm, ts, gW, st);
+        adj_sweeps_r<kStencilExt, JFA_CHAR_CONSERVATIVE>(riemann, W, lam, G, prm, ts, gW, GF, st);
+    else adj_sweeps_r<kStencilExt, JFA_PRIMITIVE>(riemann, W, lam, G, prm, ts, gW, GF, st);
 }
 
 }  // namespace jfa
