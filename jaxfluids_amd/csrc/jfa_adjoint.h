@@ -1291,7 +1291,7 @@ __device__ __forceinline__ void char_cons_window_vjp(const double* __restrict__ 
 // value (3/2 / T - 1 / (T + C)).
 __device__ __forceinline__ double law_slope(double T, double value, const Law& l) {
     if (l.kind == JFA_LAW_SUTHERLAND) return value * (1.5 / T - 1.0 / (T + l.param));
-    return l.param == 0.0 ? 0.0 : l.param * value / T;
+    return l.param == 0.0 ? 0.0 : l.param * fdiv(value, T);
 }
 
 // VJP of the dissipative flux (jfa_dissipative.h) of the face whose right cell is cr, for the
@@ -1374,10 +1374,11 @@ __device__ __forceinline__ void dissipative_face_vjp(const double* __restrict__ 
         TRb += 0.5 * Tfb;
     }
     // T = p / (rho R)
-    gl[4] += TLb / (s.wl[0] * prm.R);
-    gl[0] -= TLb * s.TL / s.wl[0];
-    gr[4] += TRb / (s.wr[0] * prm.R);
-    gr[0] -= TRb * s.TR / s.wr[0];
+    const double tl = TLb * rcp(s.wl[0]), tr = TRb * rcp(s.wr[0]), iR = rcp(prm.R);
+    gl[4] += tl * iR;
+    gl[0] -= tl * s.TL;
+    gr[4] += tr * iR;
+    gr[0] -= tr * s.TR;
 }
 
 // ------------------------------------------------------------------ kernels
@@ -2001,7 +2002,7 @@ __global__ __launch_bounds__(kBlock) void adj_dissip_cell_kernel(const double* _
     const int64_t ncell = (int64_t)G.n[0] * G.n[1] * G.n[2];
     if (!flat_index(ncell, G.n[1], G.n[2], c[0], c[1], c[2])) return;
     const int64_t idx = ((int64_t)c[0] * G.n[1] + c[1]) * G.n[2] + c[2];
-    const int64_t b = wrapped_index(G, c, 0), fs = G.fs;
+    const int64_t b = cell_index(G, c), fs = G.fs;
     double g[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, x[9] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     const double lc[5] = {ld(lam, b), ld(lam, fs + b), ld(lam, 2 * fs + b), ld(lam, 3 * fs + b), ld(lam, 4 * fs + b)};
 #pragma unroll
@@ -2009,10 +2010,10 @@ __global__ __launch_bounds__(kBlock) void adj_dissip_cell_kernel(const double* _
         if (!G.active[A]) continue;
 #pragma unroll
         for (int side = 0; side < 2; ++side) {  // 0: lower face (c is its right cell), 1: upper face
-            int cr[3] = {c[0], c[1], c[2]}, co[3] = {c[0], c[1], c[2]};
+            int cr[3] = {c[0], c[1], c[2]};
             cr[A] += side;
-            co[A] += side ? 1 : -1;  // the face's other cell
-            const int64_t bo = wrapped_index(G, co, 0);
+            // the face's other cell
+            const int64_t bo = b + (side ? offset_up(G, A, c[A], 0) : offset_down(G, A, c[A], 0));
             double mu[5], gl[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, gr[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, Gt[2][3];
             const double sc = ts * G.one_dx[A];
 #pragma unroll

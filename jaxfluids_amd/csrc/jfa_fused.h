@@ -42,7 +42,7 @@ constexpr int kMarchBlock = 256;
 // common options as constants).  The plain convective variants are held to two waves per SIMD so that
 // nothing spills; the common ones fit three by themselves.  The others need the registers: with the
 // loads ahead the dissipative variants fall to one wave per SIMD (128^3 viscous PRIMITIVE, us per
-// stage: 474 ahead, 388 at the top of the step).
+// stage: 474 ahead, 388 at the top of the step) and neither do they carry states (10 registers more).
 template <int VAR, int RIEMANN, bool DISS, bool FLIM>
 constexpr bool kPlainMarch = !(DISS || FLIM || VAR == JFA_CHAR_CONSERVATIVE || RIEMANN == kFluxSplit);
 
@@ -72,8 +72,8 @@ JFA_WAVES_PER_EU((kPlainMarch<VAR, RIEMANN, DISS, FLIM> ? 2 : 1)) void march_ker
     constexpr bool cons_win = (VAR == JFA_CONSERVATIVE || VAR == JFA_CHAR_CONSERVATIVE);
     constexpr int NW = Win<STENCIL>::n, H = Win<STENCIL>::h;
     const T* __restrict__ src = cons_win ? U : W;
-    constexpr bool CARRY = RIEMANN != kFluxSplit && kCarry<VAR, STENCIL>;
     constexpr bool AHEAD = kPlainMarch<VAR, RIEMANN, DISS, FLIM>;
+    constexpr bool CARRY = AHEAD && kCarry<VAR, STENCIL>;
     double win[NW][5], nxt[5], carry[5];
 #pragma unroll
     for (int k = 0; k < NW; ++k)
@@ -122,6 +122,8 @@ JFA_WAVES_PER_EU((kPlainMarch<VAR, RIEMANN, DISS, FLIM> ? 2 : 1)) void march_ker
                                                               Fn, carry);
         if constexpr (DISS) {
             cr[A] = a + 1;
+            JFA_OPAQUE(cr[O]);  // keeps the neighbours' addresses out of the loop's registers
+            JFA_OPAQUE(cr[IN]);
             dissipative_face<T, A>(W, G, prm, cr, Fn);
         }
 #pragma unroll
