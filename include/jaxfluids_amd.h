@@ -250,6 +250,12 @@ int jfa_rk3_stage(void* U, const void* U_n, const void* rhs, void* W, const jfa_
                   const jfa_scheme* scheme, int32_t stage, const double* dt_dev, double dt_host,
                   void* stream);
 
+/* jfa_rk3_stage of U into U_out, and prim(U_out) into W_out; the halos of U_out and W_out are copies of
+ * those of U and W.  The outputs must not overlap the inputs. */
+int jfa_rk3_stage_into(const void* W, const void* U, const void* U_n, const void* rhs, void* W_out, void* U_out,
+                       const jfa_grid* grid, const jfa_scheme* scheme, int32_t stage, const double* dt_dev,
+                       double dt_host, void* stream);
+
 /* Face-halo fill of W and U = cons(W) in the halos for PERIODIC / ZEROGRADIENT / SYMMETRY;
  * bc[6] in the order east, west, north, south, top, bottom (JFA_BC_*).
  * Replaces HaloManager.perform_halo_update_material (halos/halo_manager.py:146-234) ->

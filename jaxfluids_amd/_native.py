@@ -101,6 +101,7 @@ SIGNATURES = {
     "jfa_compute_rhs": (_I32, [_P, _P, _PG, _PS, _D, _P, _P, _SZ, _P]),
     "jfa_rhs_workspace_bytes": (_SZ, [_PG, _I32]),
     "jfa_rk3_stage": (_I32, [_P, _P, _P, _P, _PG, _PS, _I32, _P, _D, _P]),
+    "jfa_rk3_stage_into": (_I32, [_P, _P, _P, _P, _P, _P, _PG, _PS, _I32, _P, _D, _P]),
     "jfa_halo_update": (_I32, [_P, _P, _PG, _PI32, _D, _I32, _P]),
     "jfa_edge_halo_update": (_I32, [_P, _P, _PG, _PI32, _D, _I32, _P]),
     "jfa_compute_dt": (_I32, [_P, _PG, _D, _D, _D, _I32, ctypes.POINTER(JfaTransport), _P, _P, _P]),

@@ -148,20 +148,12 @@ __global__ __launch_bounds__(kBlock) void flux_xi_kernel(const T* __restrict__ W
 // ------------------------------------------------------------------ RK3 stage
 
 template <class T>
-__global__ __launch_bounds__(kBlock) void rk3_stage_kernel(T* __restrict__ U, const T* __restrict__ Un,
-                                                           const T* __restrict__ rhs, T* __restrict__ W, Geo G,
-                                                           int stage, const double* __restrict__ dt_dev,
-                                                           double dt_host, Params prm) {
-    const int64_t plane = (int64_t)G.n[1] * G.n[2];
-    int c0i, c1i, c2i;
-    if (!flat_index((int64_t)G.n[0] * plane, G.n[1], G.n[2], c0i, c1i, c2i)) return;
-    const int64_t t = (int64_t)c1i * G.n[2] + c2i;
-    const int64_t b = (int64_t)(c0i + G.off[0]) * G.s[0] + (int64_t)(c1i + G.off[1]) * G.s[1] + (c2i + G.off[2]);
-    const int64_t ncell = (int64_t)G.n[0] * plane;
-    const int64_t ro = (int64_t)c0i * plane + t;
+__device__ __forceinline__ void stage_cell(const T* U, const T* __restrict__ Un, const T* __restrict__ rhs, T* U_out,
+                                           T* __restrict__ W_out,
+                                           const Geo& G, int64_t b, int64_t ro, int64_t ncell, int stage, double dt,
+                                           const Params& prm) {
     double c0, c1, m;
     rk3_coeffs(stage, c0, c1, m);
-    const double dt = dt_dev ? dt_dev[0] : dt_host;
     const double ts = dt * m;  // RK3.py:60
     double u[5], w[5];
 #pragma unroll
@@ -174,27 +166,76 @@ __global__ __launch_bounds__(kBlock) void rk3_stage_kernel(T* __restrict__ U, co
     prim_from_cons(u, prm, w);
 #pragma unroll
     for (int i = 0; i < 5; ++i) {
-        U[i * G.fs + b] = static_cast<T>(u[i]);
-        W[i * G.fs + b] = static_cast<T>(w[i]);
+        U_out[i * G.fs + b] = static_cast<T>(u[i]);
+        W_out[i * G.fs + b] = static_cast<T>(w[i]);
     }
 }
 
-// ------------------------------------------------------------------ halos
-// One thread per face-halo cell of one face location.  W halo from the retrieve slice
-// (boundary_condition.py:564-595), U halo = cons(W halo) (outer/material.py:248-250).
+// U is updated in place: the one pointer is both source and destination, a cell reads before it writes.
 template <class T>
-__global__ __launch_bounds__(kBlock) void halo_kernel(T* __restrict__ W, T* __restrict__ U, Geo G, int axis,
-                                                      int high, int bc, Params prm) {
+__global__ __launch_bounds__(kBlock) void rk3_stage_kernel(T* U, const T* __restrict__ Un,
+                                                           const T* __restrict__ rhs, T* __restrict__ W, Geo G,
+                                                           int stage, const double* __restrict__ dt_dev,
+                                                           double dt_host, Params prm) {
+    const int64_t ncell = (int64_t)G.n[0] * G.n[1] * G.n[2];
+    int c0, c1, c2;
+    if (!flat_index(ncell, G.n[1], G.n[2], c0, c1, c2)) return;
+    const int64_t b = (int64_t)(c0 + G.off[0]) * G.s[0] + (int64_t)(c1 + G.off[1]) * G.s[1] + (c2 + G.off[2]);
+    const int64_t ro = ((int64_t)c0 * G.n[1] + c1) * G.n[2] + c2;
+    stage_cell<T>(U, Un, rhs, U, W, G, b, ro, ncell, stage, dt_dev ? dt_dev[0] : dt_host, prm);
+}
+
+// The same from one pair of buffers into another, one thread per buffer cell; the cells around the
+// interior are copied.  Bound: memory (five arrays of the interior, four of the halos).  In place of a
+// copy of each buffer and the update of the copies: 100 x 90 x 80 with 5 halo cells FP64, us per
+// stage: 34 against 19 + 19 + 28.
+template <class T>
+__global__ __launch_bounds__(kBlock) void rk3_stage_into_kernel(const T* __restrict__ W, const T* __restrict__ U,
+                                                                const T* __restrict__ Un,
+                                                                const T* __restrict__ rhs, T* __restrict__ W_out,
+                                                                T* __restrict__ U_out, Geo G, int stage,
+                                                                const double* __restrict__ dt_dev, double dt_host,
+                                                                Params prm) {
+    int c0, c1, c2;
+    if (!flat_index(G.fs, G.B[1], G.B[2], c0, c1, c2)) return;
+    const int64_t b = ((int64_t)c0 * G.B[1] + c1) * G.B[2] + c2;
+    c0 -= G.off[0];
+    c1 -= G.off[1];
+    c2 -= G.off[2];
+    if (c0 < 0 || c0 >= G.n[0] || c1 < 0 || c1 >= G.n[1] || c2 < 0 || c2 >= G.n[2]) {
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+            W_out[i * G.fs + b] = W[i * G.fs + b];
+            U_out[i * G.fs + b] = U[i * G.fs + b];
+        }
+        return;
+    }
+    const int64_t ncell = (int64_t)G.n[0] * G.n[1] * G.n[2];
+    const int64_t ro = ((int64_t)c0 * G.n[1] + c1) * G.n[2] + c2;
+    stage_cell<T>(U, Un, rhs, U_out, W_out, G, b, ro, ncell, stage, dt_dev ? dt_dev[0] : dt_host, prm);
+}
+
+// ------------------------------------------------------------------ halos
+// One thread per face-halo cell, grid.y over the faces of the active axes.  W halo from the retrieve
+// slice (boundary_condition.py:564-595), U halo = cons(W halo) (outer/material.py:248-250).  All faces in
+// one launch: a face's halo cells are copies of interior cells only, so the faces do not wait for one
+// another (100 x 90 x 80, 5 halo cells, us: 11 in one launch, 29 in six).
+template <class T>
+__global__ __launch_bounds__(kBlock) void halo_kernel(T* __restrict__ W, T* __restrict__ U, Geo G, BC6 bcs,
+                                                      Params prm) {
+    int axis = 0, faces = blockIdx.y;  // the (blockIdx.y)-th face of the active axes: high, low per axis
+    while (!G.active[axis] || faces >= 2) {
+        if (G.active[axis]) faces -= 2;
+        ++axis;
+    }
+    const int high = faces == 0;
+    const int bc = bcs.t[2 * axis + faces];
     // halo slab: nh along axis, interior along the others
     int ext[3];
     for (int i = 0; i < 3; ++i) ext[i] = i == axis ? G.nh : G.n[i];
     const int64_t total = (int64_t)ext[0] * ext[1] * ext[2];
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= total) return;
     int c[3];
-    c[2] = (int)(t % ext[2]);
-    c[1] = (int)((t / ext[2]) % ext[1]);
-    c[0] = (int)(t / ((int64_t)ext[1] * ext[2]));
+    if (!flat_index(total, ext[1], ext[2], c[0], c[1], c[2])) return;
     const int m = c[axis];  // 0..nh-1 within the slab
     const int N = G.n[axis], nh = G.nh;
     int dst, src;
@@ -490,6 +531,29 @@ int jfa_rk3_stage(void* U, const void* U_n, const void* rhs, void* W, const jfa_
     return check_launch();
 }
 
+int jfa_rk3_stage_into(const void* W, const void* U, const void* U_n, const void* rhs, void* W_out, void* U_out,
+                       const jfa_grid* grid, const jfa_scheme* scheme, int32_t stage, const double* dt_dev,
+                       double dt_host, void* stream) {
+    Geo G;
+    int rc = make_geo(grid, G);
+    if (rc) return rc;
+    rc = check_scheme(scheme);
+    if (rc) return rc;
+    if (!W || !U || !rhs || !W_out || !U_out || stage < 0 || stage > 2 || (stage > 0 && !U_n)) return JFA_EINVAL;
+    if (W_out == W || U_out == U) return JFA_EINVAL;
+    const dim3 g = flat_grid(G.fs);
+    hipStream_t st = (hipStream_t)stream;
+    if (scheme->dtype == JFA_F32)
+        hipLaunchKernelGGL((rk3_stage_into_kernel<float>), g, dim3(kBlock), 0, st, (const float*)W, (const float*)U,
+                           (const float*)U_n, (const float*)rhs, (float*)W_out, (float*)U_out, G, stage, dt_dev,
+                           dt_host, make_params(scheme));
+    else
+        hipLaunchKernelGGL((rk3_stage_into_kernel<double>), g, dim3(kBlock), 0, st, (const double*)W,
+                           (const double*)U, (const double*)U_n, (const double*)rhs, (double*)W_out, (double*)U_out, G,
+                           stage, dt_dev, dt_host, make_params(scheme));
+    return check_launch();
+}
+
 int jfa_halo_update(void* W, void* U, const jfa_grid* grid, const int32_t bc[6], double gamma, int32_t dtype,
                     void* stream) {
     Geo G;
@@ -499,27 +563,29 @@ int jfa_halo_update(void* W, void* U, const jfa_grid* grid, const int32_t bc[6],
     if (dtype != JFA_F64 && dtype != JFA_F32) return JFA_EUNSUPPORTED;
     hipStream_t st = (hipStream_t)stream;
     // halo_slices.py:66-73 face order east, west, north, south, top, bottom
+    BC6 b6;
+    int faces = 0;
+    int64_t total = 0;
     for (int loc = 0; loc < 6; ++loc) {
         const int axis = loc / 2;
+        b6.t[loc] = bc[loc];
         if (!G.active[axis]) continue;
-        const int b = bc[loc];
-        if (b < 0 || b > 2) return JFA_EUNSUPPORTED;
-        if (G.nh > G.n[axis] && b != JFA_BC_ZEROGRADIENT) return JFA_EINVAL;
-        const int high = (loc % 2) == 0;
-        int64_t total = G.nh;
+        if (bc[loc] < 0 || bc[loc] > 2) return JFA_EUNSUPPORTED;
+        if (G.nh > G.n[axis] && bc[loc] != JFA_BC_ZEROGRADIENT) return JFA_EINVAL;
+        ++faces;
+        int64_t slab = G.nh;
         for (int i = 0; i < 3; ++i)
-            if (i != axis) total *= G.n[i];
-        dim3 g((unsigned)((total + kBlock - 1) / kBlock));
-        if (dtype == JFA_F32)
-            hipLaunchKernelGGL((halo_kernel<float>), g, dim3(kBlock), 0, st, (float*)W, (float*)U, G, axis, high, b,
-                               gas_params(gamma));
-        else
-            hipLaunchKernelGGL((halo_kernel<double>), g, dim3(kBlock), 0, st, (double*)W, (double*)U, G, axis, high,
-                               b, gas_params(gamma));
-        rc = check_launch();
-        if (rc) return rc;
+            if (i != axis) slab *= G.n[i];
+        if (slab > total) total = slab;
     }
-    return JFA_OK;
+    if (!faces) return JFA_OK;
+    dim3 g((unsigned)((total + kBlock - 1) / kBlock), (unsigned)faces);
+    if (dtype == JFA_F32)
+        hipLaunchKernelGGL((halo_kernel<float>), g, dim3(kBlock), 0, st, (float*)W, (float*)U, G, b6, gas_params(gamma));
+    else
+        hipLaunchKernelGGL((halo_kernel<double>), g, dim3(kBlock), 0, st, (double*)W, (double*)U, G, b6,
+                           gas_params(gamma));
+    return check_launch();
 }
 
 int jfa_edge_halo_update(void* W, void* U, const jfa_grid* grid, const int32_t bc[6], double gamma,

@@ -115,10 +115,9 @@ class SimulationManager:
         for stage in range(self.time_integrator.no_stages):
             rhs, _, _ = self.space_solver.compute_rhs(U, W, physical_timestep_size=dt)
             W_new = torch.empty_like(W)
-            W_new.copy_(W)
             integ = self.time_integrator.perform_stage_integration(
                 integ, rhs, init, dt, stage, self.equation_information, self.domain_information,
-                self.material_manager.get_gamma(), primitives_out=W_new)
+                self.material_manager.get_gamma(), primitives_out=W_new, primitives=W)
             U = integ.euler_buffers.conservatives
             W, U = self.halo_manager.perform_halo_update_material(W_new, 0.0, self.halo_manager.fill_edge_halos_material,
                                                                   False, U, inplace=True)

@@ -63,14 +63,18 @@ class RungeKutta3(TimeIntegrator):
     def perform_stage_integration(self, integration_buffers: IntegrationBuffers, rhs_buffers: IntegrationBuffers,
                                   initial_stage_buffers: IntegrationBuffers, physical_timestep_size, stage: int,
                                   equation_information=None, domain_information=None, gamma: float = None,
-                                  primitives_out: torch.Tensor = None) -> IntegrationBuffers:
+                                  primitives_out: torch.Tensor = None,
+                                  primitives: torch.Tensor = None) -> IntegrationBuffers:
         """Stage blend + update on the GPU (time_integrator.py:108-227, jfa_rk3_stage).
 
         ``physical_timestep_size`` may be a float or a device scalar tensor.  When
         ``primitives_out`` is given the kernel also writes prim(U) of the interior into it
-        (simulation_manager.py:943-944), saving a separate conversion pass.
+        (simulation_manager.py:943-944), saving a separate conversion pass; with ``primitives``
+        (those of the given conservatives, contiguous like them) it writes the halos too, copies of
+        theirs, so neither buffer is copied beforehand.
         """
-        U = integration_buffers.euler_buffers.conservatives.clone()
+        U_in = integration_buffers.euler_buffers.conservatives
+        U = U_in.clone() if primitives is None else torch.empty_like(U_in)
         Un = initial_stage_buffers.euler_buffers.conservatives if stage > 0 else None
         rhs = rhs_buffers.euler_buffers.conservatives.contiguous()
         if domain_information is None or gamma is None:
@@ -79,9 +83,15 @@ class RungeKutta3(TimeIntegrator):
         dt_dev, dt_host = _dt_args(physical_timestep_size)
         scheme = _native.make_scheme("PRIMITIVE", "WENO5-JS", "HLLC", "EINFELDT", "ARITHMETIC",
                                      _native.dtype_code(U), gamma, precision.get_spatial_stencil_eps())
-        rc = _native.load().jfa_rk3_stage(_native.ptr(U), _native.ptr(Un), _native.ptr(rhs), _native.ptr(W),
-                                          domain_information.grid, scheme, int(stage), dt_dev, dt_host,
-                                          _native.stream_ptr())
+        if primitives is None:
+            rc = _native.load().jfa_rk3_stage(_native.ptr(U), _native.ptr(Un), _native.ptr(rhs), _native.ptr(W),
+                                              domain_information.grid, scheme, int(stage), dt_dev, dt_host,
+                                              _native.stream_ptr())
+        else:
+            rc = _native.load().jfa_rk3_stage_into(_native.ptr(primitives), _native.ptr(U_in), _native.ptr(Un),
+                                                   _native.ptr(rhs), _native.ptr(W), _native.ptr(U),
+                                                   domain_information.grid, scheme, int(stage), dt_dev, dt_host,
+                                                   _native.stream_ptr())
         _native.check(rc, "jfa_rk3_stage")
         return IntegrationBuffers(EulerIntegrationBuffers(U))
 
