@@ -62,6 +62,7 @@ class SimulationManager:
         self._bufs = None
         self._graph = None
         self._graph_key = None
+        self._dt_host = None
         self.wall_clock_times = []
 
     # ------------------------------------------------------------------ buffers
@@ -83,17 +84,28 @@ class SimulationManager:
         return self._bufs
 
     # ------------------------------------------------------------------ stages
+    def _stage_call(self, W: torch.Tensor):
+        """jfa_rk3_stage_fused with the arguments that the stages of a step share: on a small grid the
+        three stages run on the GPU for as long as building these for each takes (1000 cells: 7 us)."""
+        b = self._bufs
+        scheme = self.convective_flux_solver.scheme(_native.dtype_code(W), self.space_solver.transport)
+        eps = precision.get_eps() if W.dtype == torch.float64 else float(torch.finfo(torch.float32).eps)
+        cfl = float(self.numerical_setup.conservatives.time_integration.CFL)
+        grid, bcs = self.domain_information.grid, self.halo_manager.bc_array
+        ws, ws_bytes, stream = b["ws"].data_ptr(), b["ws"].numel(), _native.stream_ptr()
+        fused = _native.load().jfa_rk3_stage_fused
+
+        def call(W_in, U_in, U_n, W_out, U_out, stage: int, dt: torch.Tensor, dt_next: Optional[torch.Tensor] = None):
+            rc = fused(W_in.data_ptr(), U_in.data_ptr(), None if U_n is None else U_n.data_ptr(), W_out.data_ptr(),
+                       U_out.data_ptr(), grid, scheme, bcs, stage, dt.data_ptr(), 0.0, cfl, eps,
+                       None if dt_next is None else dt_next.data_ptr(), ws, ws_bytes, stream)
+            _native.check(rc, "jfa_rk3_stage_fused")
+
+        return call
+
     def _fused_stage(self, W_in, U_in, U_n, W_out, U_out, stage: int, dt: torch.Tensor,
                      dt_next: Optional[torch.Tensor] = None) -> None:
-        b = self._bufs
-        scheme = self.convective_flux_solver.scheme(_native.dtype_code(W_in), self.space_solver.transport)
-        eps = precision.get_eps() if W_in.dtype == torch.float64 else float(torch.finfo(torch.float32).eps)
-        cfl = float(self.numerical_setup.conservatives.time_integration.CFL)
-        rc = _native.load().jfa_rk3_stage_fused(
-            _native.ptr(W_in), _native.ptr(U_in), _native.ptr(U_n), _native.ptr(W_out), _native.ptr(U_out),
-            self.domain_information.grid, scheme, self.halo_manager.bc_array, int(stage), _native.ptr(dt), 0.0,
-            cfl, eps, _native.ptr(dt_next), _native.ptr(b["ws"]), b["ws"].numel(), _native.stream_ptr())
-        _native.check(rc, "jfa_rk3_stage_fused")
+        self._stage_call(W_in)(W_in, U_in, U_n, W_out, U_out, int(stage), dt, dt_next)
 
     def do_runge_kutta_stages(self, primitives: torch.Tensor, conservatives: torch.Tensor, dt: torch.Tensor,
                               dt_next: Optional[torch.Tensor] = None):
@@ -103,11 +115,12 @@ class SimulationManager:
         if self.fused:
             b = self._ensure_buffers(primitives)
             (Wb, Ub), (Wc, Uc) = b["B"], b["C"]
-            self._fused_stage(primitives, conservatives, None, Wb, Ub, 0, dt)
-            self._fused_stage(Wb, Ub, conservatives, Wc, Uc, 1, dt)
+            stage = self._stage_call(primitives)
+            stage(primitives, conservatives, None, Wb, Ub, 0, dt)
+            stage(Wb, Ub, conservatives, Wc, Uc, 1, dt)
             # U_out may alias U_n: each cell reads U_n[c] before writing U_out[c], and no cell
             # reads U_n in the halos.
-            self._fused_stage(Wc, Uc, conservatives, primitives, conservatives, 2, dt, dt_next)
+            stage(Wc, Uc, conservatives, primitives, conservatives, 2, dt, dt_next)
             return primitives, conservatives
         W, U = primitives, conservatives
         init = IntegrationBuffers(EulerIntegrationBuffers(U))
@@ -165,12 +178,20 @@ class SimulationManager:
         dt = tcv.physical_timestep_size
         if not isinstance(dt, torch.Tensor):
             dt = torch.full((1,), float(dt), dtype=torch.float64, device=W.device)
-        dt_used = float(dt.item())
+        # the step overwrites dt: its value goes to the host ahead of the step's kernels, and the wait for
+        # it follows their launch (the GPU would idle for a round trip of 12 us otherwise)
+        if self._dt_host is None:
+            self._dt_host = (torch.empty(1, dtype=torch.float64, pin_memory=True), torch.cuda.Event())
+        dt_host, copied = self._dt_host
+        dt_host.copy_(dt.reshape(1), non_blocking=True)
+        copied.record()
         if self.use_graph and self.fused:
             # the replayed step reads and writes dt in place
             self._capture(W, U, dt).replay()
         else:
             W, U = self._step_kernels(W, U, dt)
+        copied.synchronize()
+        dt_used = float(dt_host)
         tcv = tcv._replace(physical_simulation_time=tcv.physical_simulation_time + dt_used,
                            simulation_step=tcv.simulation_step + 1, physical_timestep_size=dt)
         return JaxFluidsBuffers(MaterialFieldBuffers(U, W, mf.temperature), tcv)
