@@ -349,6 +349,10 @@ int jfa_adjoint_set_march_min_waves(int64_t waves);
 int jfa_rk3_stage_vjp(const void* W_in, const void* lam_out, void* lam_in, void* lam_n, const jfa_grid* grid,
                       const jfa_scheme* scheme, const int32_t bc[6], int32_t stage, double dt, void* workspace,
                       size_t workspace_bytes, void* stream);
+/* The same, but the interior of lam_in (set & 1) and of lam_n (set & 2) is written instead of added to. */
+int jfa_rk3_stage_vjp_set(const void* W_in, const void* lam_out, void* lam_in, void* lam_n, const jfa_grid* grid,
+                          const jfa_scheme* scheme, const int32_t bc[6], int32_t stage, double dt, int32_t set,
+                          void* workspace, size_t workspace_bytes, void* stream);
 
 /* ---- Ensembles of independent 2-D domains (z inactive), advanced by one launch per RK3
  * stage for all cases together.  Each case is a (5, Nx+2nh, Ny+2nh, 1) block inside pooled

@@ -217,8 +217,10 @@ class FixedDtStepper:
         if nb == 0:
             raise _native.JFAError("invalid grid for the adjoint")
         self._aws = torch.empty(nb, dtype=torch.uint8, device=self.device)
-        self._lam = [e(), e(), e()]
-        self._lam_out = [e(), e()]
+        # cotangents of the stages' states; the kernels write interiors only, halos stay zero
+        z = lambda: torch.zeros(self.shape, dtype=torch.float64, device=self.device)
+        self._lam = [z(), z()]
+        self._lam_out = [z(), z()]
         self._nvjp = 0
         self._work = (e(), e())
         self._pools: Dict[str, torch.Tensor] = {}
@@ -289,11 +291,12 @@ class FixedDtStepper:
         """Frees the rollout buffers kept by `buffers`."""
         self._pools.clear()
 
-    def _vjp(self, W_in, lam_out, lam_in, lam_n, k) -> None:
+    def _vjp(self, W_in, lam_out, lam_in, lam_n, k, fresh: int) -> None:
+        """Adds to lam_in and lam_n, or writes them (fresh & 1, fresh & 2)."""
         P = _native.ptr
-        rc = _native.load().jfa_rk3_stage_vjp(P(W_in), P(lam_out), P(lam_in), P(lam_n), self.grid, self.scheme,
-                                              self.bc, k, self.dt_value, P(self._aws), self._aws.numel(),
-                                              _native.stream_ptr())
+        rc = _native.load().jfa_rk3_stage_vjp_set(P(W_in), P(lam_out), P(lam_in), P(lam_n), self.grid, self.scheme,
+                                                  self.bc, k, self.dt_value, fresh, P(self._aws), self._aws.numel(),
+                                                  _native.stream_ptr())
         _native.check(rc, "jfa_rk3_stage_vjp")
 
     def step_vjp(self, W: torch.Tensor, U: torch.Tensor, lam: torch.Tensor,
@@ -308,18 +311,15 @@ class FixedDtStepper:
         else:
             self._stage(W, U, None, Wb, Ub, 0)
             self._stage(Wb, Ub, U, Wc, Uc, 1)
-        l2, l1, l0 = self._lam
-        for t in (l2, l1, l0):
-            t.zero_()  # fill kernels (graph-safe), halos stay zero
-        self._vjp(Wc, lam, l2, l0, 2)
-        self._vjp(Wb, l2, l1, l0, 1)
-        self._vjp(W, l1, l0, None, 0)
+        l2, l1 = self._lam
         # two output buffers in turn: the returned cotangent is the next call's input
         out = self._lam_out[self._nvjp % 2]
-        if out is lam:
+        if out.data_ptr() == lam.data_ptr():
             out = self._lam_out[(self._nvjp + 1) % 2]
         self._nvjp += 1
-        out.copy_(l0)
+        self._vjp(Wc, lam, l2, out, 2, 3)
+        self._vjp(Wb, l2, l1, out, 1, 1)
+        self._vjp(W, l1, out, None, 0, 0)
         return out
 
     # -- rollouts

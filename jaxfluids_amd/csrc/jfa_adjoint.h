@@ -1738,10 +1738,12 @@ __global__ __launch_bounds__(kAdjBlock) void adj_face_kernel(const double* __res
 
 // Cell pass along A: lanes over the columns (buffer order of IN), chunk blockIdx.y owns the cells
 // [-3 + y L, -3 + (y + 1) L) of its columns and walks the centres that reach them, variable blockIdx.z.
+// A centre's loads are issued before the previous centre's store.  first: gW is written, not added to;
+// the halo cells along A are this pass's alone and always written.
 template <int A, int IN, int STENCIL>
 __global__ __launch_bounds__(kAdjBlock) void adj_cell_march_kernel(const double* __restrict__ W,
                                                                    const double* __restrict__ GF, Geo G, FaceIdx F,
-                                                                   Params prm, int L, double* __restrict__ gW) {
+                                                                   Params prm, int L, int first, double* __restrict__ gW) {
     constexpr int O = 3 - A - IN;
     const int col = blockIdx.x * kAdjBlock + threadIdx.x;
     const int io = col / G.n[IN], iin = col - io * G.n[IN];
@@ -1760,31 +1762,42 @@ __global__ __launch_bounds__(kAdjBlock) void adj_cell_march_kernel(const double*
     double x[5], acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int k = 0; k < 4; ++k) x[k + 1] = ld(W, b0 + (int64_t)(ca - 2 + k) * sa);
+    // of centre c: its upper window cell, its states' cotangents and the old sum of the cell it completes
+    auto load = [&](int c, double& w, double& vh, double& vl, double& g) {
+        w = ld(W, b0 + (int64_t)(c + 2) * sa);
+        vh = c < N ? ld(GF, fl + (c + 1) * fsA) : 0.0;
+        vl = c >= 0 ? ld(GF, fr + c * fsA) : 0.0;
+        const int o = c - 2;
+        g = !first && o >= o0 && o >= 0 && o < N ? ld(gW, b0 + (int64_t)o * sa) : 0.0;
+    };
     auto put = [&](int cell, double v) {
         if (cell >= o0 && cell < o1) {
-            double* p = gW + b0 + (int64_t)cell * sa;
-            JFA_ACCESS(p, sizeof(double));
-            *p += v;
+            JFA_ACCESS(gW + b0 + (int64_t)cell * sa, sizeof(double));
+            gW[b0 + (int64_t)cell * sa] = v;
         }
     };
+    double w, vh, vl, g;
+    load(ca, w, vh, vl, g);
     for (int c = ca; c <= cb; ++c) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) x[k] = x[k + 1];
-        x[4] = ld(W, b0 + (int64_t)(c + 2) * sa);
-        const double vh = c < N ? ld(GF, fl + (c + 1) * fsA) : 0.0;
-        const double vl = c >= 0 ? ld(GF, fr + c * fsA) : 0.0;
+        x[4] = w;
+        const double h = vh, l = vl, old = g;
+        load(c < cb ? c + 1 : c, w, vh, vl, g);
         double o[5];
-        weno5_cell_vjp<STENCIL>(x[0], x[1], x[2], x[3], x[4], prm.eps_z, prm.eps_js, vh, vl, o);
+        weno5_cell_vjp<STENCIL>(x[0], x[1], x[2], x[3], x[4], prm.eps_z, prm.eps_js, h, l, o);
 #pragma unroll
         for (int k = 0; k < 5; ++k) acc[k] += o[k];
-        put(c - 2, acc[0]);
+        put(c - 2, old + acc[0]);
 #pragma unroll
         for (int k = 0; k < 4; ++k) acc[k] = acc[k + 1];
         acc[4] = 0.0;
     }
-    if (cb == N) {
+    if (cb == N) {  // cells N - 1 .. N + 2 are complete
+        const double old = !first && N - 1 >= o0 && N - 1 < o1 ? ld(gW, b0 + (int64_t)(N - 1) * sa) : 0.0;
+        put(N - 1, old + acc[0]);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) put(N - 1 + k, acc[k]);
+        for (int k = 1; k < 4; ++k) put(N - 1 + k, acc[k]);
     }
 }
 
@@ -1794,7 +1807,7 @@ __global__ __launch_bounds__(kAdjBlock) void adj_cell_march_kernel(const double*
 template <int A, int STENCIL>
 __global__ __launch_bounds__(kAdjBlock) void adj_cell_lane_kernel(const double* __restrict__ W,
                                                                   const double* __restrict__ GF, Geo G, FaceIdx F,
-                                                                  Params prm, int waves_per_row, int64_t nwaves,
+                                                                  Params prm, int waves_per_row, int64_t nwaves, int first,
                                                                   double* __restrict__ gW) {
     constexpr int P = A == 0 ? 1 : 0;
     constexpr int Q = A == 2 ? 1 : 2;
@@ -1828,7 +1841,7 @@ __global__ __launch_bounds__(kAdjBlock) void adj_cell_lane_kernel(const double* 
     if (vwave && lane >= 2 && lane < 62 && c <= N + 2) {
         double* p = gW + b0 + (int64_t)c * sa;
         JFA_ACCESS(p, sizeof(double));
-        *p += s;
+        *p = first || c < 0 || c >= N ? s : *p + s;
     }
 }
 
@@ -2063,7 +2076,7 @@ __device__ __forceinline__ void xbar_gather(const double* __restrict__ X, const 
 
 // Per interior cell: halo^T, (dW/dU)^T and the stage blend.
 __device__ __forceinline__ void halo_gather(const double* __restrict__ gW, const Geo& G, const BC6& bc,
-                                            const int c[3], int64_t b, double g[5]) {
+                                            const int c[3], int64_t b, int reach, double g[5]) {
     const int nh = G.nh;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
@@ -2075,13 +2088,13 @@ __device__ __forceinline__ void halo_gather(const double* __restrict__ gW, const
         const int tl = bc.t[2 * a + 1], th = bc.t[2 * a];
         // low halo (west/south/bottom) -- transpose of halo_scatter's low side
         if (tl == JFA_BC_PERIODIC) {
-            if (ci >= N - nh)
+            if (ci >= N - reach)
                 for (int i = 0; i < 5; ++i) g[i] += ld(gW, i * G.fs + bc0 + (int64_t)(ci - N + nh) * sa);
         } else if (tl == JFA_BC_ZEROGRADIENT) {
             if (ci == 0)
-                for (int m = 0; m < nh; ++m)
+                for (int m = nh - reach; m < nh; ++m)
                     for (int i = 0; i < 5; ++i) g[i] += ld(gW, i * G.fs + bc0 + (int64_t)m * sa);
-        } else if (ci < nh) {
+        } else if (ci < reach) {
             for (int i = 0; i < 5; ++i) {
                 const double h = ld(gW, i * G.fs + bc0 + (int64_t)(nh - 1 - ci) * sa);
                 g[i] += i == a + 1 ? -h : h;
@@ -2089,13 +2102,13 @@ __device__ __forceinline__ void halo_gather(const double* __restrict__ gW, const
         }
         // high halo (east/north/top)
         if (th == JFA_BC_PERIODIC) {
-            if (ci < nh)
+            if (ci < reach)
                 for (int i = 0; i < 5; ++i) g[i] += ld(gW, i * G.fs + bc0 + (int64_t)(N + nh + ci) * sa);
         } else if (th == JFA_BC_ZEROGRADIENT) {
             if (ci == N - 1)
-                for (int m = 0; m < nh; ++m)
+                for (int m = 0; m < reach; ++m)
                     for (int i = 0; i < 5; ++i) g[i] += ld(gW, i * G.fs + bc0 + (int64_t)(N + nh + m) * sa);
-        } else if (ci >= N - nh) {
+        } else if (ci >= N - reach) {
             for (int i = 0; i < 5; ++i) {
                 const double h = ld(gW, i * G.fs + bc0 + (int64_t)(N + nh + (N - 1 - ci)) * sa);
                 g[i] += i == a + 1 ? -h : h;
@@ -2108,7 +2121,8 @@ template <int UNUSED = 0>  // a template, so the translation units that include 
 __global__ __launch_bounds__(kBlock) void adj_update_kernel(const double* __restrict__ W,
                                                             const double* __restrict__ lam,
                                                             const double* __restrict__ gW, Geo G, Params prm,
-                                                            BC6 bc, double c0, double c1, double* __restrict__ lam_in,
+                                                            BC6 bc, double c0, double c1, int reach, int set,
+                                                            double* __restrict__ lam_in,
                                                             double* __restrict__ lam_n,
                                                             const double* __restrict__ X) {
     int c[3];
@@ -2122,19 +2136,21 @@ __global__ __launch_bounds__(kBlock) void adj_update_kernel(const double* __rest
         w[i] = ld(W, i * fs + b);
         l[i] = ld(lam, i * fs + b);
     }
-    halo_gather(gW, G, bc, c, b, g);
+    halo_gather(gW, G, bc, c, b, reach, g);
     if (X) xbar_gather(X, G, c, g);
     prim_vjp(w, g, prm, gu);
 #pragma unroll
     for (int i = 0; i < 5; ++i) {
         JFA_ACCESS(lam_in + i * fs + b, sizeof(double));
-        lam_in[i * fs + b] += c0 * l[i] + gu[i];
+        const double v = c0 * l[i] + gu[i];
+        lam_in[i * fs + b] = set & 1 ? v : lam_in[i * fs + b] + v;
     }
     if (lam_n) {
 #pragma unroll
         for (int i = 0; i < 5; ++i) {
             JFA_ACCESS(lam_n + i * fs + b, sizeof(double));
-            lam_n[i * fs + b] += c1 * l[i];
+            const double v = c1 * l[i];
+            lam_n[i * fs + b] = set & 2 ? v : lam_n[i * fs + b] + v;
         }
     }
 }
@@ -2189,11 +2205,13 @@ static inline int64_t max_faces(const Geo& G) {
     return m;
 }
 
-// The two passes along axis A.  Chunks of the marching cell pass: the longest of 64, 32, 16, 8 (4
-// centres more than cells each) that still fills the device four times over.
+// The two passes along axis A (first: of the sweep's first axis).  Chunks of the marching cell pass: the
+// longest of 64, 32, 16, 8, 4 (4 centres more than cells each) that still fills the device four times
+// over; a small grid is bound by the chain of a chunk's loads (256^2, us along x: 14 with
+// 8 cells and each centre's loads after the last one's store, 9.5 with 4 and the loads ahead).
 template <int A, int IN, int STENCIL, int RIEMANN>
 static void launch_two_pass(const double* W, const double* lam, const Geo& G, const Params& prm, double ts, double* GF,
-                            double* gW, hipStream_t st) {
+                            int first, double* gW, hipStream_t st) {
     const FaceIdx F = face_extents(G, A);
     hipLaunchKernelGGL((adj_face_kernel<A, STENCIL, RIEMANN>), flat_grid(F.nface), dim3(kAdjBlock), 0, st, W, lam, G, F,
                        prm, ts, GF);
@@ -2203,15 +2221,15 @@ static void launch_two_pass(const double* W, const double* lam, const Geo& G, co
         const int64_t nwaves = (int64_t)waves_per_row * G.n[P] * G.n[Q];
         const int64_t blocks = (nwaves + kAdjBlock / 64 - 1) / (kAdjBlock / 64);
         hipLaunchKernelGGL((adj_cell_lane_kernel<A, STENCIL>), dim3((unsigned)blocks, 5), dim3(kAdjBlock), 0, st, W, GF,
-                           G, F, prm, waves_per_row, nwaves, gW);
+                           G, F, prm, waves_per_row, nwaves, first, gW);
     } else {
         constexpr int O = 3 - A - IN;
         const int64_t cols = (int64_t)G.n[IN] * G.n[O], cells = G.n[A] + 6;
         int L = 64;
-        while (L > 8 && 5 * ((cols + 63) / 64) * ((cells + L - 1) / L) < 16384) L /= 2;
+        while (L > 4 && 5 * ((cols + 63) / 64) * ((cells + L - 1) / L) < 16384) L /= 2;
         hipLaunchKernelGGL((adj_cell_march_kernel<A, IN, STENCIL>),
                            dim3((unsigned)((cols + kAdjBlock - 1) / kAdjBlock), (unsigned)((cells + L - 1) / L), 5),
-                           dim3(kAdjBlock), 0, st, W, GF, G, F, prm, L, gW);
+                           dim3(kAdjBlock), 0, st, W, GF, G, F, prm, L, first, gW);
     }
 }
 
@@ -2222,17 +2240,22 @@ static void adj_sweeps(const double* W, const double* lam, const Geo& G, const P
                        double* GF, hipStream_t st) {
     const int IN = innermost_axis(G);
     if constexpr (kTwoPass<VAR, STENCIL, RIEMANN>) {
-        if (IN == 0) {
-            launch_two_pass<0, 0, STENCIL, RIEMANN>(W, lam, G, prm, ts, GF, gW, st);
-        } else if (IN == 1) {
-            if (G.active[0]) launch_two_pass<0, 1, STENCIL, RIEMANN>(W, lam, G, prm, ts, GF, gW, st);
-            launch_two_pass<1, 1, STENCIL, RIEMANN>(W, lam, G, prm, ts, GF, gW, st);
-        } else {
-            if (G.active[0]) launch_two_pass<0, 2, STENCIL, RIEMANN>(W, lam, G, prm, ts, GF, gW, st);
-            if (G.active[1]) launch_two_pass<1, 2, STENCIL, RIEMANN>(W, lam, G, prm, ts, GF, gW, st);
-            launch_two_pass<2, 2, STENCIL, RIEMANN>(W, lam, G, prm, ts, GF, gW, st);
+        int first = 1;
+        if (IN > 0 && G.active[0]) {
+            if (IN == 1) launch_two_pass<0, 1, STENCIL, RIEMANN>(W, lam, G, prm, ts, GF, first, gW, st);
+            else launch_two_pass<0, 2, STENCIL, RIEMANN>(W, lam, G, prm, ts, GF, first, gW, st);
+            first = 0;
         }
+        if (IN == 2 && G.active[1]) {
+            launch_two_pass<1, 2, STENCIL, RIEMANN>(W, lam, G, prm, ts, GF, first, gW, st);
+            first = 0;
+        }
+        if (IN == 0) launch_two_pass<0, 0, STENCIL, RIEMANN>(W, lam, G, prm, ts, GF, first, gW, st);
+        else if (IN == 1) launch_two_pass<1, 1, STENCIL, RIEMANN>(W, lam, G, prm, ts, GF, first, gW, st);
+        else launch_two_pass<2, 2, STENCIL, RIEMANN>(W, lam, G, prm, ts, GF, first, gW, st);
     } else {
+        const int64_t nz = 5 * G.fs, zb = (nz + kBlock - 1) / kBlock;
+        hipLaunchKernelGGL(adj_zero_kernel<0>, dim3((unsigned)(zb < 4096 ? zb : 4096)), dim3(kBlock), 0, st, gW, nz);
         const int64_t min_waves = adjoint_march_min_waves();
         for (int A = 0; A < IN; ++A) {
             if (!G.active[A]) continue;

@@ -21,12 +21,15 @@ int jfa_adjoint_set_march_min_waves(int64_t waves) {
     return JFA_OK;
 }
 
+// the schemes of kTwoPass
+static bool two_pass(const jfa_scheme* s) {
+    return s->recon_var == JFA_PRIMITIVE && s->riemann < JFA_FS_ROE &&
+           (s->stencil == JFA_WENO5_JS || s->stencil == JFA_WENO5_Z);
+}
+
 static size_t vjp_workspace_bytes(const Geo& G, const jfa_scheme* scheme) {
     size_t n = (size_t)(5 * G.fs);
-    // face cotangents of one axis (kTwoPass); without a scheme, enough for any
-    if (!scheme || (scheme->recon_var == JFA_PRIMITIVE && scheme->riemann < JFA_FS_ROE &&
-                    (scheme->stencil == JFA_WENO5_JS || scheme->stencil == JFA_WENO5_Z)))
-        n += (size_t)(10 * max_faces(G));
+    if (!scheme || two_pass(scheme)) n += (size_t)(10 * max_faces(G));  // face cotangents of one axis
     if (scheme && scheme->transport && (scheme->transport->viscous || scheme->transport->heat))
         n += (size_t)9 * ((size_t)G.n[0] * G.n[1] * G.n[2]);  // X: transverse-derivative cotangent sums
     return n * sizeof(double);
@@ -41,6 +44,13 @@ size_t jfa_stage_vjp_workspace_bytes(const jfa_grid* grid, const jfa_scheme* sch
 int jfa_rk3_stage_vjp(const void* W_in, const void* lam_out, void* lam_in, void* lam_n, const jfa_grid* grid,
                       const jfa_scheme* scheme, const int32_t bc[6], int32_t stage, double dt, void* workspace,
                       size_t workspace_bytes, void* stream) {
+    return jfa_rk3_stage_vjp_set(W_in, lam_out, lam_in, lam_n, grid, scheme, bc, stage, dt, 0, workspace,
+                                 workspace_bytes, stream);
+}
+
+int jfa_rk3_stage_vjp_set(const void* W_in, const void* lam_out, void* lam_in, void* lam_n, const jfa_grid* grid,
+                          const jfa_scheme* scheme, const int32_t bc[6], int32_t stage, double dt, int32_t set,
+                          void* workspace, size_t workspace_bytes, void* stream) {
     Geo G;
     int rc = make_geo(grid, G);
     if (rc) return rc;
@@ -63,6 +73,7 @@ int jfa_rk3_stage_vjp(const void* W_in, const void* lam_out, void* lam_in, void*
     if (!W_in || !lam_out || !lam_in || !bc || !workspace || stage < 0 || stage > 2 || (stage > 0 && !lam_n))
         return JFA_EINVAL;
     if (lam_in == lam_out || lam_n == lam_out || (stage > 0 && lam_n == lam_in)) return JFA_EINVAL;
+    if (set < 0 || set > 3) return JFA_EINVAL;
     if (!(dt > 0.0) || workspace_bytes < vjp_workspace_bytes(G, scheme)) return JFA_EINVAL;
     BC6 b6;
     for (int f = 0; f < 6; ++f) {
@@ -84,8 +95,6 @@ int jfa_rk3_stage_vjp(const void* W_in, const void* lam_out, void* lam_in, void*
     const int64_t nz = 5 * G.fs;
     double* X = prm.dissip ? gW + nz : nullptr;  // written whole by the cell kernel: no clearing
     double* GF = gW + nz + (prm.dissip ? 9 * (int64_t)G.n[0] * G.n[1] * G.n[2] : 0);
-    const int64_t zb = (nz + kBlock - 1) / kBlock;
-    hipLaunchKernelGGL(adj_zero_kernel<0>, dim3((unsigned)(zb < 4096 ? zb : 4096)), dim3(kBlock), 0, st, gW, nz);
     const double* W = static_cast<const double*>(W_in);
     const double* lam = static_cast<const double*>(lam_out);
     const int var = fsplit ? JFA_PRIMITIVE : scheme->recon_var;  // flux splitting: the primitive window
@@ -114,6 +123,7 @@ int jfa_rk3_stage_vjp(const void* W_in, const void* lam_out, void* lam_in, void*
     }
     const int64_t ncell = (int64_t)G.n[0] * G.n[1] * G.n[2];
     hipLaunchKernelGGL(adj_update_kernel<0>, flat_grid(ncell), dim3(kBlock), 0, st, W, lam, gW, G, prm, b6, c0, c1,
+                       two_pass(scheme) ? 3 : G.nh, set,
                        static_cast<double*>(lam_in), stage > 0 ? static_cast<double*>(lam_n) : nullptr, X);
     return check_launch();
 }

@@ -6,10 +6,11 @@ A lane wave owns 60 cells of a row with its three halo cells a side (54 cells fi
 a second, 114 fill two), a marching chunk 8 cells of a column on grids this small (10 cells fill two
 chunks, 11 start a third); 3 cells are the fewest that a periodic axis with three halo cells takes.
 """
+import numpy as np
 import pytest
 
 from oracle import jxf_oracle as o
-from test_emu_adjoint import FACES, emu  # noqa: F401 - emu: fixture
+from test_emu_adjoint import FACES, emu, run_vjp, smooth_state  # noqa: F401 - emu: fixture
 from test_torch_stage import _compare
 
 PERIODIC = ("PERIODIC",) * 6
@@ -25,3 +26,35 @@ def test_matches_autograd(emu, cells, bcs, stencil, riemann):  # noqa: F811
     s = o.Setup(gamma=1.4, stencil=stencil, variable="PRIMITIVE", riemann=riemann, signal_speed="EINFELDT",
                 bcs=dict(zip(FACES, bcs)))
     _compare(emu, dom, s, 1, "march", sum(cells), sum(cells) + 1)
+
+
+@pytest.mark.parametrize("variable", ["PRIMITIVE", "CHAR-PRIMITIVE"])
+@pytest.mark.parametrize("cells, nh, bcs", [((7, 9, 1), 5, WALLS), ((6, 1, 5), 4, PERIODIC), ((9, 1, 1), 3, WALLS)])
+def test_written_equals_added_to_zero(emu, cells, nh, bcs, variable):  # noqa: F811
+    """jfa_rk3_stage_vjp_set into NaN, from a workspace of NaN, is jfa_rk3_stage_vjp into zeros: nothing is
+    read that the call has not written (more halo cells than the stencil reaches, too)."""
+    from jaxfluids_amd import _native
+
+    fn = emu.jfa_rk3_stage_vjp_set
+    fn.restype, fn.argtypes = _native.SIGNATURES["jfa_rk3_stage_vjp_set"]
+    dom = o.Domain(cells, nh=nh)
+    s = o.Setup(gamma=1.4, stencil="WENO5-Z", variable=variable, riemann="HLLC", signal_speed="EINFELDT",
+                frozen_state="ARITHMETIC", bcs=dict(zip(FACES, bcs)))
+    W = np.ascontiguousarray(o.create_buffers(smooth_state(dom, sum(cells)), dom, s)[0])
+    lam = np.zeros((5,) + dom.shape)
+    lam[dom.interior] = np.random.default_rng(sum(cells)).standard_normal((5,) + cells)
+    added = run_vjp(emu, dom, s, W, lam, 2, 1e-3)
+    grid = _native.make_grid(dom.cells, nh, dom.dx)
+    scheme = _native.make_scheme(s.variable, s.stencil, s.riemann, s.signal_speed, s.frozen_state, _native.F64, s.gamma,
+                                 s.eps_stencil)
+    ws = np.full(emu.jfa_stage_vjp_workspace_bytes(grid, scheme) // 8, np.nan)
+    written = [np.full_like(lam, np.nan), np.full_like(lam, np.nan)]
+    args = [a.ctypes.data for a in (W, lam, *written)] + [grid, scheme, _native.bc_array(s.bcs), 2, 1e-3]
+    emu.emu_clear_ranges()
+    for a in (W, lam, *written, ws):
+        emu.emu_add_range(a.ctypes.data, a.nbytes)
+    assert fn(*args, 3, ws.ctypes.data, ws.nbytes, None) == 0
+    assert emu.emu_violations() == 0, hex(emu.emu_first_violation())
+    for a, w in zip(added, written):
+        assert np.array_equal(a[dom.interior], w[dom.interior])
+    assert fn(*args, 4, ws.ctypes.data, ws.nbytes, None) == _native.JFA_EINVAL
