@@ -1294,17 +1294,15 @@ __device__ __forceinline__ double law_slope(double T, double value, const Law& l
     return l.param == 0.0 ? 0.0 : l.param * fdiv(value, T);
 }
 
-// VJP of the dissipative flux (jfa_dissipative.h) of the face whose right cell is cr, for the
-// cotangent m of the face flux.  Adds the cotangents of the left and right cells' primitives to
+// VJP of the dissipative flux (jfa_dissipative.h) of a face with state s, for the cotangent m of
+// the face flux.  Adds the cotangents of the left and right cells' primitives to
 // gl, gr and returns Gt[j][k], j-th axis i != AXIS (ascending), velocity component k: the face
 // sends +Gt to u_k at L + e_i and R + e_i and -Gt to u_k at L - e_i and R - e_i (the transverse
 // central derivatives).  The clamp of T_f <= 0 has zero derivative.
 template <int AXIS>
-__device__ __forceinline__ void dissipative_face_vjp(const double* __restrict__ W, const Geo& G, const Params& prm,
-                                                     const int cr[3], const double m[5], double gl[5], double gr[5],
-                                                     double Gt[2][3]) {
-    DissState s;
-    dissipative_state<double, AXIS>(W, G, prm, cr, s);
+__device__ __forceinline__ void dissipative_state_vjp(const DissState& s, const Geo& G, const Params& prm,
+                                                      const double m[5], double gl[5], double gr[5],
+                                                      double Gt[2][3]) {
     double mub = 0.0, Tfb = 0.0, TLb = 0.0, TRb = 0.0;
 #pragma unroll
     for (int j = 0; j < 2; ++j)
@@ -2001,13 +1999,56 @@ __device__ __forceinline__ int64_t interior_flat(const Geo& G, const int c[3]) {
     return ((int64_t)w[0] * G.n[1] + w[1]) * G.n[2] + w[2];
 }
 
+// Face state between cell c (primitives wc, temperature Tc, transverse derivatives dc[i][k] of u_k) and its
+// neighbour bo along AXIS, above it (side 1) or below; up, down: offsets to the neighbours of either cell
+// across AXIS.  The values are those of dissipative_state.
+template <int AXIS>
+__device__ __forceinline__ void dissipative_state_of_cell(const double* __restrict__ W, const Geo& G,
+                                                          const Params& prm, const double wc[5], double Tc,
+                                                          const double (&dc)[3][3], int64_t bo, int side,
+                                                          const int64_t up[3], const int64_t down[3], DissState& s) {
+    double wn[5];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        wn[i] = ld(W, i * G.fs + bo);
+        s.wl[i] = side ? wc[i] : wn[i];
+        s.wr[i] = side ? wn[i] : wc[i];
+    }
+    const double Tn = wn[4] / (wn[0] * prm.R);
+    s.TL = side ? Tc : Tn;
+    s.TR = side ? Tn : Tc;
+    s.Tf = 0.5 * (s.TL + s.TR);
+    s.clamped = s.Tf <= 0.0;
+    if (s.clamped) s.Tf = 2.220446049250313e-16;  // source_term_solver.py:301 (precision eps)
+    s.mu = viscosity(s.Tf, prm);
+    if (!(prm.dissip & 1)) return;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        if (!G.active[i]) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) s.g[k][i] = 0.0;
+        } else if (i == AXIS) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) s.g[k][i] = (s.wr[1 + k] - s.wl[1 + k]) * G.one_dx[i];
+        } else {
+            double u[3], d[3];
+            load_velocity(W, G.fs, bo + up[i], u);
+            load_velocity(W, G.fs, bo + down[i], d);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) s.g[k][i] = 0.5 * (dc[i][k] + (u[k] - d[k]) * (0.5 * G.one_dx[i]));
+        }
+    }
+}
+
 // Dissipative part, one thread per interior cell c: the VJPs of both faces of c along every
 // active axis (periodic: the forward's faces 0 and n evaluate the same wrapped cells, so their
 // cotangents combine into ts (lam_R - lam_L) / dx with wrapped lam), so c owns its whole
 // dissipative cotangent, added to gW, and the sum X[3 i + k](c) of the transverse-derivative
 // cotangents Gt of its faces (interior layout, ncell per field), gathered by adj_update_kernel.
+// What the six faces share (c's state, temperature and transverse derivatives) is formed once: bound by
+// loads through L1, 160 a cell against 324 with each face on its own (128^3, us: 265 and 302).
 template <int UNUSED = 0>
-__global__ __launch_bounds__(kBlock) void adj_dissip_cell_kernel(const double* __restrict__ W,
+__global__ __launch_bounds__(kBlock) JFA_WAVES_PER_EU(3) void adj_dissip_cell_kernel(const double* __restrict__ W,
                                                                  const double* __restrict__ lam, Geo G, Params prm,
                                                                  double ts, double* __restrict__ gW,
                                                                  double* __restrict__ X) {
@@ -2017,16 +2058,31 @@ __global__ __launch_bounds__(kBlock) void adj_dissip_cell_kernel(const double* _
     const int64_t idx = ((int64_t)c[0] * G.n[1] + c[1]) * G.n[2] + c[2];
     const int64_t b = cell_index(G, c), fs = G.fs;
     double g[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, x[9] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    const double lc[5] = {ld(lam, b), ld(lam, fs + b), ld(lam, 2 * fs + b), ld(lam, 3 * fs + b), ld(lam, 4 * fs + b)};
+    double lc[5], wc[5], dc[3][3];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        lc[i] = ld(lam, i * fs + b);
+        wc[i] = ld(W, i * fs + b);
+    }
+    const double Tc = wc[4] / (wc[0] * prm.R);
+    int64_t up[3], down[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        up[i] = offset_up(G, i, c[i], 0);
+        down[i] = offset_down(G, i, c[i], 0);
+        if (!G.active[i] || !(prm.dissip & 1)) continue;
+        double u[3], d[3];
+        load_velocity(W, fs, b + up[i], u);
+        load_velocity(W, fs, b + down[i], d);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) dc[i][k] = (u[k] - d[k]) * (0.5 * G.one_dx[i]);
+    }
 #pragma unroll
     for (int A = 0; A < 3; ++A) {
         if (!G.active[A]) continue;
 #pragma unroll
         for (int side = 0; side < 2; ++side) {  // 0: lower face (c is its right cell), 1: upper face
-            int cr[3] = {c[0], c[1], c[2]};
-            cr[A] += side;
-            // the face's other cell
-            const int64_t bo = b + (side ? offset_up(G, A, c[A], 0) : offset_down(G, A, c[A], 0));
+            const int64_t bo = b + (side ? up[A] : down[A]);  // the face's other cell
             double mu[5], gl[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, gr[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, Gt[2][3];
             const double sc = ts * G.one_dx[A];
 #pragma unroll
@@ -2034,9 +2090,17 @@ __global__ __launch_bounds__(kBlock) void adj_dissip_cell_kernel(const double* _
                 const double lo = ld(lam, i * fs + bo);
                 mu[i] = side ? sc * (lo - lc[i]) : sc * (lc[i] - lo);
             }
-            if (A == 0) dissipative_face_vjp<0>(W, G, prm, cr, mu, gl, gr, Gt);
-            else if (A == 1) dissipative_face_vjp<1>(W, G, prm, cr, mu, gl, gr, Gt);
-            else dissipative_face_vjp<2>(W, G, prm, cr, mu, gl, gr, Gt);
+            DissState s;
+            if (A == 0) {
+                dissipative_state_of_cell<0>(W, G, prm, wc, Tc, dc, bo, side, up, down, s);
+                dissipative_state_vjp<0>(s, G, prm, mu, gl, gr, Gt);
+            } else if (A == 1) {
+                dissipative_state_of_cell<1>(W, G, prm, wc, Tc, dc, bo, side, up, down, s);
+                dissipative_state_vjp<1>(s, G, prm, mu, gl, gr, Gt);
+            } else {
+                dissipative_state_of_cell<2>(W, G, prm, wc, Tc, dc, bo, side, up, down, s);
+                dissipative_state_vjp<2>(s, G, prm, mu, gl, gr, Gt);
+            }
 #pragma unroll
             for (int i = 0; i < 5; ++i) g[i] += side ? gl[i] : gr[i];
             int j = 0;
