@@ -348,7 +348,16 @@ __global__ __launch_bounds__(1024) void dt_from_parts_kernel(const double* __res
     const int nq = dissip ? 3 : 1;
     for (int q = 0; q < nq; ++q) {
         double v = 0.0;
-        for (int i = threadIdx.x; i < n; i += blockDim.x) v = nan_max(v, part[q * n + i]);
+        for (int i = threadIdx.x; i < n; i += 8 * blockDim.x) {  // eight loads in flight (25000 partials, us: 18 -> 12)
+            double x[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int j = i + k * (int)blockDim.x;
+                x[k] = j < n ? part[q * n + j] : 0.0;
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v = nan_max(v, x[k]);
+        }
         for (int o = 32; o > 0; o >>= 1) v = nan_max(v, __shfl_xor(v, o, 64));
         if ((threadIdx.x & 63) == 0) sm[q][threadIdx.x >> 6] = v;
     }
