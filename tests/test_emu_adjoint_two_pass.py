@@ -2,9 +2,10 @@
 adj_cell_lane_kernel of jfa_adjoint.h) at the edges of their waves and chunks, through the host build
 of the library, against torch autograd of the stage (test_torch_stage, at its tolerance).
 
-A lane wave owns 60 cells of a row with its three halo cells a side (54 cells fill one wave, 55 start
-a second, 114 fill two), a marching chunk 8 cells of a column on grids this small (10 cells fill two
-chunks, 11 start a third); 3 cells are the fewest that a periodic axis with three halo cells takes.
+A lane wave owns 60 positions of the rows, which lie one after another with their three halo cells a
+side (rows of 54 cells fill a wave each, rows of 55 and 114 end inside one), a marching chunk 4 cells of
+a column on grids this small (10 cells fill four chunks, 11 start a fifth); 3 cells are the fewest that
+a periodic axis with three halo cells takes.
 """
 import numpy as np
 import pytest
