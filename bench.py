@@ -274,7 +274,7 @@ def bench_ensemble(steps: int, warmup: int, ncases: int = 64, seed: int = 0, nh:
         "with_interpolation_limiter": limited,
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
-                     "kernel": "batch2d_stage_kernel", "avg_stage_ms": round(kern_ms / len(ev), 4)},
+                     "kernel": "batch2d_walk_kernel", "avg_stage_ms": round(kern_ms / len(ev), 4)},
     }
 
 
@@ -603,7 +603,7 @@ def main():
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": measured_stage_figure(args.n, args.dtype, args.variable, args.nh),
-                     "kernel": "RK3 stage (jfa_rk3_stage_fused: x/y marching sweeps + z sweep with update)",
+                     "kernel": "RK3 stage (jfa_rk3_stage_fused: x marching sweep + y and z faces with update)",
                      "avg_stage_ms": round(tot_ms / len(events), 4),
                      "alg_bytes_per_cell_stage": round(sum(byt) / 3, 2)},
     }
