@@ -291,7 +291,8 @@ int jfa_prim_from_cons(const void* U, void* W, int64_t ncells, double gamma, int
  * (accumulated in the reference's axis order), stage blend and update, W = prim(U), and the
  * face-halo fill of W and U for the boundary types bc[6] -- the work of jfa_compute_rhs +
  * jfa_rk3_stage + jfa_halo_update without face-flux arrays: one marching sweep per active
- * non-innermost axis and one innermost-axis sweep that finishes the stage.
+ * non-innermost axis and one innermost-axis sweep that finishes the stage (the common schemes: the
+ * last two in one kernel).
  * If dt_next_dev is non-NULL, the CFL time step of the new state (as jfa_compute_dt, with
  * `cfl` and `eps`) is written to dt_next_dev[0]; it may alias dt_dev.
  * W_out/U_out must not alias W_in/U_in; U_out may alias U_n.

@@ -2003,43 +2003,21 @@ __device__ __forceinline__ int64_t interior_flat(const Geo& G, const int c[3]) {
 
 // Face state between cell c (primitives wc, temperature Tc, transverse derivatives dc[i][k] of u_k) and its
 // neighbour bo along AXIS, above it (side 1) or below; up, down: offsets to the neighbours of either cell
-// across AXIS.  The values are those of dissipative_state.
+// across AXIS.
 template <int AXIS>
 __device__ __forceinline__ void dissipative_state_of_cell(const double* __restrict__ W, const Geo& G,
                                                           const Params& prm, const double wc[5], double Tc,
                                                           const double (&dc)[3][3], int64_t bo, int side,
                                                           const int64_t up[3], const int64_t down[3], DissState& s) {
-    double wn[5];
+    double wn[5], dn[3][3];
 #pragma unroll
-    for (int i = 0; i < 5; ++i) {
-        wn[i] = ld(W, i * G.fs + bo);
-        s.wl[i] = side ? wc[i] : wn[i];
-        s.wr[i] = side ? wn[i] : wc[i];
-    }
-    const double Tn = wn[4] / (wn[0] * prm.R);
-    s.TL = side ? Tc : Tn;
-    s.TR = side ? Tn : Tc;
-    s.Tf = 0.5 * (s.TL + s.TR);
-    s.clamped = s.Tf <= 0.0;
-    if (s.clamped) s.Tf = 2.220446049250313e-16;  // source_term_solver.py:301 (precision eps)
-    s.mu = viscosity(s.Tf, prm);
-    if (!(prm.dissip & 1)) return;
+    for (int i = 0; i < 5; ++i) wn[i] = ld(W, i * G.fs + bo);
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        if (!G.active[i]) {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) s.g[k][i] = 0.0;
-        } else if (i == AXIS) {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) s.g[k][i] = (s.wr[1 + k] - s.wl[1 + k]) * G.one_dx[i];
-        } else {
-            double u[3], d[3];
-            load_velocity(W, G.fs, bo + up[i], u);
-            load_velocity(W, G.fs, bo + down[i], d);
-#pragma unroll
-            for (int k = 0; k < 3; ++k) s.g[k][i] = 0.5 * (dc[i][k] + (u[k] - d[k]) * (0.5 * G.one_dx[i]));
-        }
-    }
+    for (int i = 0; i < 3; ++i)
+        if (i != AXIS && G.active[i] && (prm.dissip & 1)) velocity_derivative(W, G, i, bo, up[i], down[i], dn[i]);
+    const double Tn = temperature(wn, prm);
+    if (side) dissipative_state_between<AXIS>(G, prm, wc, Tc, dc, wn, Tn, dn, s);
+    else dissipative_state_between<AXIS>(G, prm, wn, Tn, dn, wc, Tc, dc, s);
 }
 
 // Dissipative part, one thread per interior cell c: the VJPs of both faces of c along every
@@ -2066,18 +2044,13 @@ __global__ __launch_bounds__(kBlock) JFA_WAVES_PER_EU(3) void adj_dissip_cell_ke
         lc[i] = ld(lam, i * fs + b);
         wc[i] = ld(W, i * fs + b);
     }
-    const double Tc = wc[4] / (wc[0] * prm.R);
+    const double Tc = temperature(wc, prm);
     int64_t up[3], down[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         up[i] = offset_up(G, i, c[i], 0);
         down[i] = offset_down(G, i, c[i], 0);
-        if (!G.active[i] || !(prm.dissip & 1)) continue;
-        double u[3], d[3];
-        load_velocity(W, fs, b + up[i], u);
-        load_velocity(W, fs, b + down[i], d);
-#pragma unroll
-        for (int k = 0; k < 3; ++k) dc[i][k] = (u[k] - d[k]) * (0.5 * G.one_dx[i]);
+        if (G.active[i] && (prm.dissip & 1)) velocity_derivative(W, G, i, b, up[i], down[i], dc[i]);
     }
 #pragma unroll
     for (int A = 0; A < 3; ++A) {

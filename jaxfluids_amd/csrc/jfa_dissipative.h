@@ -11,15 +11,28 @@
 //   tau_k = mu (g[AXIS][k] + g[k][AXIS]) (active k), tau_AXIS += mu2 sum_k g[k][k]
 //   F[1+k] += -tau_k;  F[4] += -sum_k tau_k u_f,k + q,  q = -kappa(T_f) (T_R - T_L)/dx,
 //   kappa = cp mu / Pr (PRANDTL) or its own POWER / SUTHERLAND law      (material.py:103-124)
-// On periodic domains the accesses wrap onto the interior (the halos and edge halos there are
-// periodic copies); otherwise (prm.diss_halos) they read the buffer's face and edge halos, which
-// the stage's halo scatter and edge-halo fill wrote.
+// The two cells are those of the convective window.  On periodic domains their transverse neighbours wrap
+// onto the interior (the edge halos there may be unwritten; they would be periodic copies); otherwise
+// (prm.diss_halos) they are read from the buffer's face and edge halos, which the stage's halo scatter
+// and edge-halo fill wrote.
 #pragma once
 
 #include "jfa_common.h"
 
 namespace jfa {
 
+// A series coefficient, with SCALAR in scalar registers and formed where it is used.  The compiler copies
+// each into vector registers before its fma, or keeps them all in scalar registers around a loop and
+// spills others for it: a viscous sweep takes 223 VGPRs so and 177 with SCALAR.  Where many faces stand
+// in one block the asm keeps them from being interleaved: the reverse's cell kernel spills with SCALAR
+// (128^3, us: 331 against 250).
+template <bool SCALAR>
+__device__ __forceinline__ double coef(double c) {
+    if constexpr (!SCALAR) return c;
+    long long bits = __double_as_longlong(c);
+    JFA_OPAQUE_S(bits);
+    return __longlong_as_double(bits);
+}
 // x^p as exp(p log x) with the logarithm in two doubles: log x = k ln 2 + log m, m in [sqrt(1/2), sqrt(2)),
 // log m = 2 artanh(s), s = (m - 1)/(m + 1) (its series to s^27); exp by its series on half a binade, the first
 // terms summed with their errors.  86 instructions against 226 for pow(x, p), which a viscous face
@@ -28,6 +41,7 @@ namespace jfa {
 // extended precision on the GPU, 4e5 values each of x in [e^-300, e^300] and p of -0.7 .. 3: below
 // 0.57 ulp, mean 0.25 (pow: 1.33 and up to 0.35).
 constexpr double kLn2Hi = 0x1.62e42fefa0000p-1, kLn2Lo = 0x1.cf79abc9e3b3ap-40;
+template <bool SCALAR>
 __device__ __forceinline__ double power(double x, double p) {
 #pragma clang fp contract(off)
     int k;
@@ -40,19 +54,19 @@ __device__ __forceinline__ double power(double x, double p) {
     const double s = f * r;
     const double sl = r * fma(-s, dl, fma(-s, d, f));
     const double z = s * s;
-    double P = 1.0 / 27.0;
-    P = fma(P, z, 1.0 / 25.0);
-    P = fma(P, z, 1.0 / 23.0);
-    P = fma(P, z, 1.0 / 21.0);
-    P = fma(P, z, 1.0 / 19.0);
-    P = fma(P, z, 1.0 / 17.0);
-    P = fma(P, z, 1.0 / 15.0);
-    P = fma(P, z, 1.0 / 13.0);
-    P = fma(P, z, 1.0 / 11.0);
-    P = fma(P, z, 1.0 / 9.0);
-    P = fma(P, z, 1.0 / 7.0);
-    P = fma(P, z, 1.0 / 5.0);
-    P = fma(P, z, 1.0 / 3.0);
+    double P = coef<SCALAR>(1.0 / 27.0);
+    P = fma(P, z, coef<SCALAR>(1.0 / 25.0));
+    P = fma(P, z, coef<SCALAR>(1.0 / 23.0));
+    P = fma(P, z, coef<SCALAR>(1.0 / 21.0));
+    P = fma(P, z, coef<SCALAR>(1.0 / 19.0));
+    P = fma(P, z, coef<SCALAR>(1.0 / 17.0));
+    P = fma(P, z, coef<SCALAR>(1.0 / 15.0));
+    P = fma(P, z, coef<SCALAR>(1.0 / 13.0));
+    P = fma(P, z, coef<SCALAR>(1.0 / 11.0));
+    P = fma(P, z, coef<SCALAR>(1.0 / 9.0));
+    P = fma(P, z, coef<SCALAR>(1.0 / 7.0));
+    P = fma(P, z, coef<SCALAR>(1.0 / 5.0));
+    P = fma(P, z, coef<SCALAR>(1.0 / 3.0));
     const double t = s * (z * P);
     const double n1 = (double)k;
     const double A = n1 * kLn2Hi, S = s + s;
@@ -65,18 +79,18 @@ __device__ __forceinline__ double power(double x, double p) {
     const double q0 = fma(-n2, kLn2Hi, y);
     const double qr = fma(-n2, kLn2Lo, yl);
     const double q = q0 + qr, ql = qr - (q - q0);
-    double E = 1.0 / 87178291200.0;
-    E = fma(E, q, 1.0 / 6227020800.0);
-    E = fma(E, q, 1.0 / 479001600.0);
-    E = fma(E, q, 1.0 / 39916800.0);
-    E = fma(E, q, 1.0 / 3628800.0);
-    E = fma(E, q, 1.0 / 362880.0);
-    E = fma(E, q, 1.0 / 40320.0);
-    E = fma(E, q, 1.0 / 5040.0);
-    E = fma(E, q, 1.0 / 720.0);
-    E = fma(E, q, 1.0 / 120.0);
-    E = fma(E, q, 1.0 / 24.0);
-    E = fma(E, q, 1.0 / 6.0);
+    double E = coef<SCALAR>(1.0 / 87178291200.0);
+    E = fma(E, q, coef<SCALAR>(1.0 / 6227020800.0));
+    E = fma(E, q, coef<SCALAR>(1.0 / 479001600.0));
+    E = fma(E, q, coef<SCALAR>(1.0 / 39916800.0));
+    E = fma(E, q, coef<SCALAR>(1.0 / 3628800.0));
+    E = fma(E, q, coef<SCALAR>(1.0 / 362880.0));
+    E = fma(E, q, coef<SCALAR>(1.0 / 40320.0));
+    E = fma(E, q, coef<SCALAR>(1.0 / 5040.0));
+    E = fma(E, q, coef<SCALAR>(1.0 / 720.0));
+    E = fma(E, q, coef<SCALAR>(1.0 / 120.0));
+    E = fma(E, q, coef<SCALAR>(1.0 / 24.0));
+    E = fma(E, q, coef<SCALAR>(1.0 / 6.0));
     const double hq = 0.5 * q, b = hq * q, be = fma(hq, q, -b);
     const double u = q + b, w = 1.0 + u;
     const double c = fma(b * q, E + E, fma(q, ql, ql) + be);
@@ -85,19 +99,24 @@ __device__ __forceinline__ double power(double x, double p) {
     return finite ? v : (p > 0.0 ? x : __builtin_amdgcn_rcp(x));  // 0, infinity, NaN
 }
 
+template <bool SCALAR = false>
 __device__ __forceinline__ double law_value(double T, const Law& l) {
     if (l.kind == JFA_LAW_SUTHERLAND) {  // material.py:94-96, power3_2 (math/power_functions.py:29-30)
         const double x = T * l.inv_T_ref;
         return l.ref * ((l.T_ref + l.param) / (T + l.param)) * (x * sqrt(x));
     }
-    return l.param == 0.0 ? l.ref : l.ref * power(T * l.inv_T_ref, l.param);
+    return l.param == 0.0 ? l.ref : l.ref * power<SCALAR>(T * l.inv_T_ref, l.param);
 }
 
-__device__ __forceinline__ double viscosity(double T, const Params& prm) { return law_value(T, prm.mu); }
+template <bool SCALAR = false>
+__device__ __forceinline__ double viscosity(double T, const Params& prm) {
+    return law_value<SCALAR>(T, prm.mu);
+}
 
 // thermal conductivity at temperature T, where mu = viscosity(T)
+template <bool SCALAR = false>
 __device__ __forceinline__ double conductivity(double T, double mu, const Params& prm) {
-    return prm.kappa.kind == JFA_LAW_PRANDTL ? prm.kappa_fac * mu : law_value(T, prm.kappa);
+    return prm.kappa.kind == JFA_LAW_PRANDTL ? prm.kappa_fac * mu : law_value<SCALAR>(T, prm.kappa);
 }
 
 // Offsets from a cell at coordinate c along axis i to its neighbours above and below: on periodic
@@ -132,59 +151,77 @@ struct DissState {
     double g[3][3];
 };
 
-// face whose right cell has interior coordinates cr (cr[AXIS] in 0..n, the left cell is cr - e_AXIS)
+// temperature of a cell (ideal_gas.py:81-83)
+__device__ __forceinline__ double temperature(const double w[5], const Params& prm) {
+    return w[4] / (w[0] * prm.R);
+}
+
+// central derivative of the velocity along axis i at cell b, from its neighbours at the given offsets
+template <class T>
+__device__ __forceinline__ void velocity_derivative(const T* __restrict__ W, const Geo& G, int i, int64_t b, int64_t up,
+                                                    int64_t down, double d[3]) {
+    double u[3], v[3];
+    load_velocity(W, G.fs, b + up, u);
+    load_velocity(W, G.fs, b + down, v);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) d[k] = (u[k] - v[k]) * (0.5 * G.one_dx[i]);
+}
+
+// Face state along AXIS between two cells given by their primitives, temperatures and transverse velocity
+// derivatives d[i][k] = d u_k / d x_i (i != AXIS; read with viscous fluxes only).
+template <int AXIS, bool SCALAR = false>
+__device__ __forceinline__ void dissipative_state_between(const Geo& G, const Params& prm, const double wl[5],
+                                                          double TL, const double (&dl)[3][3], const double wr[5],
+                                                          double TR, const double (&dr)[3][3], DissState& s) {
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        s.wl[i] = wl[i];
+        s.wr[i] = wr[i];
+    }
+    s.TL = TL;
+    s.TR = TR;
+    s.Tf = 0.5 * (s.TL + s.TR);
+    s.clamped = s.Tf <= 0.0;
+    if (s.clamped) s.Tf = 2.220446049250313e-16;  // source_term_solver.py:301 (precision eps)
+    s.mu = viscosity<SCALAR>(s.Tf, prm);
+    if (!(prm.dissip & 1)) return;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            if (!G.active[i]) s.g[k][i] = 0.0;
+            else if (i == AXIS) s.g[k][i] = (s.wr[1 + k] - s.wl[1 + k]) * G.one_dx[i];
+            else s.g[k][i] = 0.5 * (dl[i][k] + dr[i][k]);
+        }
+}
+
+// Transverse velocity derivatives d[i][k], i != AXIS, at cell b, whose coordinates across AXIS are c's.
 template <class T, int AXIS>
-__device__ __forceinline__ void dissipative_state(const T* __restrict__ W, const Geo& G, const Params& prm,
-                                                  const int cr[3], DissState& s) {
-    const int64_t fs = G.fs;
-    // the cells beside the face; faces 0 and n of a periodic domain lie between the same two cells
-    int64_t br = cell_index(G, cr), bl = br - G.s[AXIS];
+__device__ __forceinline__ void transverse_derivatives(const T* __restrict__ W, const Geo& G, const Params& prm,
+                                                       const int c[3], int64_t b, double (&d)[3][3]) {
+    if (!(prm.dissip & 1)) return;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+        if (i != AXIS && G.active[i])
+            velocity_derivative(W, G, i, b, offset_up(G, i, c[i], prm.diss_halos), offset_down(G, i, c[i], prm.diss_halos),
+                                d[i]);
+}
+
+// Buffer indices of the cells beside the face whose right cell is cr; faces 0 and n of a periodic domain
+// lie between the same two cells.
+template <int AXIS>
+__device__ __forceinline__ void face_cells(const Geo& G, const Params& prm, const int cr[3], int64_t& bl, int64_t& br) {
+    br = cell_index(G, cr);
+    bl = br - G.s[AXIS];
     if (!prm.diss_halos) {
         const int64_t row = (int64_t)G.n[AXIS] * G.s[AXIS];
         if (cr[AXIS] == 0) bl += row;
         if (cr[AXIS] == G.n[AXIS]) br -= row;
     }
-#pragma unroll
-    for (int i = 0; i < 5; ++i) {
-        s.wl[i] = ld(W, i * fs + bl);
-        s.wr[i] = ld(W, i * fs + br);
-    }
-    s.TL = s.wl[4] / (s.wl[0] * prm.R);
-    s.TR = s.wr[4] / (s.wr[0] * prm.R);
-    s.Tf = 0.5 * (s.TL + s.TR);
-    s.clamped = s.Tf <= 0.0;
-    if (s.clamped) s.Tf = 2.220446049250313e-16;  // source_term_solver.py:301 (precision eps)
-    s.mu = viscosity(s.Tf, prm);
-    if (!(prm.dissip & 1)) return;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        if (!G.active[i]) {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) s.g[k][i] = 0.0;
-        } else if (i == AXIS) {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) s.g[k][i] = (s.wr[1 + k] - s.wl[1 + k]) * G.one_dx[i];
-        } else {
-            const double h = 0.5 * G.one_dx[i];
-            const int64_t hi = offset_up(G, i, cr[i], prm.diss_halos), lo = offset_down(G, i, cr[i], prm.diss_halos);
-            double up[3], um[3], dL[3], dR[3];
-            load_velocity(W, fs, bl + hi, up);
-            load_velocity(W, fs, bl + lo, um);
-#pragma unroll
-            for (int k = 0; k < 3; ++k) dL[k] = (up[k] - um[k]) * h;
-            load_velocity(W, fs, br + hi, up);
-            load_velocity(W, fs, br + lo, um);
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                dR[k] = (up[k] - um[k]) * h;
-                s.g[k][i] = 0.5 * (dL[k] + dR[k]);
-            }
-        }
-    }
 }
 
 // adds the dissipative flux of a face state to F
-template <int AXIS>
+template <int AXIS, bool SCALAR = false>
 __device__ __forceinline__ void dissipative_flux(const DissState& s, const Geo& G, const Params& prm, double F[5]) {
     double d4 = 0.0;
     if (prm.dissip & 1) {
@@ -205,25 +242,31 @@ __device__ __forceinline__ void dissipative_flux(const DissState& s, const Geo& 
         for (int k = 0; k < 3; ++k) F[1 + k] = F[1 + k] + (-tau[k]);
         d4 = -vel_tau;
     }
-    if (prm.dissip & 2) d4 = d4 + (-conductivity(s.Tf, s.mu, prm) * ((s.TR - s.TL) * G.one_dx[AXIS]));
+    if (prm.dissip & 2) d4 = d4 + (-conductivity<SCALAR>(s.Tf, s.mu, prm) * ((s.TR - s.TL) * G.one_dx[AXIS]));
     F[4] = F[4] + d4;
 }
 
-// adds the dissipative flux of the face whose right cell has interior coordinates cr to F
+// adds the dissipative flux of the face whose right cell has interior coordinates cr and whose cells hold
+// the primitives wl, wr to F
 template <class T, int AXIS>
 __device__ __forceinline__ void dissipative_face(const T* __restrict__ W, const Geo& G, const Params& prm,
-                                                 const int cr[3], double F[5]) {
+                                                 const int cr[3], const double wl[5], const double wr[5], double F[5]) {
+    int64_t bl, br;
+    face_cells<AXIS>(G, prm, cr, bl, br);
+    double dl[3][3], dr[3][3];
+    transverse_derivatives<T, AXIS>(W, G, prm, cr, bl, dl);
+    transverse_derivatives<T, AXIS>(W, G, prm, cr, br, dr);
     DissState s;
-    dissipative_state<T, AXIS>(W, G, prm, cr, s);
-    dissipative_flux<AXIS>(s, G, prm, F);
+    dissipative_state_between<AXIS, true>(G, prm, wl, temperature(wl, prm), dl, wr, temperature(wr, prm), dr, s);
+    dissipative_flux<AXIS, true>(s, G, prm, F);
 }
 
 // cell diffusivities for the time-step limits: nu = mu/rho, alpha = kappa/(rho cp)
 __device__ __forceinline__ void diffusivities(const double w[5], const Params& prm, double& nu, double& alpha) {
     const double T = w[4] / (w[0] * prm.R);
-    const double mu = viscosity(T, prm);
+    const double mu = viscosity<true>(T, prm);
     nu = (prm.dissip & 1) ? mu / w[0] : 0.0;
-    alpha = (prm.dissip & 2) ? conductivity(T, mu, prm) / w[0] * prm.inv_cp : 0.0;
+    alpha = (prm.dissip & 2) ? conductivity<true>(T, mu, prm) / w[0] * prm.inv_cp : 0.0;
 }
 
 }  // namespace jfa

@@ -40,15 +40,17 @@ constexpr int kMarchBlock = 256;
 // ahead, before the step's stores, so no wait covers a store (256^3 CHAR-PRIMITIVE WENO5-Z HLLC, us
 // per sweep along x / y: 507 / 589 loading at the top of the step, 433 / 476 ahead, 397 / - with the
 // common options as constants).  The plain convective variants are held to two waves per SIMD so that
-// nothing spills; the common ones fit three by themselves.  The others need the registers: with the
-// loads ahead the dissipative variants fall to one wave per SIMD (128^3 viscous PRIMITIVE, us per
-// stage: 474 ahead, 388 at the top of the step) and neither do they carry states (10 registers more).
-template <int VAR, int RIEMANN, bool DISS, bool FLIM>
-constexpr bool kPlainMarch = !(DISS || FLIM || VAR == JFA_CHAR_CONSERVATIVE || RIEMANN == kFluxSplit);
+// nothing spills; the common ones fit three by themselves.  So are the dissipative ones with a WENO5
+// stencil and HLLC or Rusanov (128^3 viscous PRIMITIVE, us per sweep: 97 loading at the top of the
+// step without carried states, 89 with both); the others need more registers and do neither.
+template <int VAR, int STENCIL, int RIEMANN, bool DISS, bool FLIM>
+constexpr bool kPlainMarch = !(FLIM || VAR == JFA_CHAR_CONSERVATIVE || RIEMANN == kFluxSplit) &&
+                             (!DISS || ((STENCIL == JFA_WENO5_JS || STENCIL == JFA_WENO5_Z) &&
+                                        (RIEMANN == JFA_HLLC || RIEMANN == JFA_RUSANOV)));
 
 template <class T, int A, int IN, int VAR, int STENCIL, int RIEMANN, bool DISS, bool FLIM, bool COMMON>
 __global__ __launch_bounds__(kMarchBlock)
-JFA_WAVES_PER_EU((kPlainMarch<VAR, RIEMANN, DISS, FLIM> ? 2 : 1)) void march_kernel(
+JFA_WAVES_PER_EU((kPlainMarch<VAR, STENCIL, RIEMANN, DISS, FLIM> ? 2 : 1)) void march_kernel(
     const T* __restrict__ W, const T* __restrict__ U, Geo G, Params prm_, int L, int rowlen, int accumulate,
     double* __restrict__ R) {
     constexpr int O = 3 - A - IN;
@@ -72,7 +74,7 @@ JFA_WAVES_PER_EU((kPlainMarch<VAR, RIEMANN, DISS, FLIM> ? 2 : 1)) void march_ker
     constexpr bool cons_win = (VAR == JFA_CONSERVATIVE || VAR == JFA_CHAR_CONSERVATIVE);
     constexpr int NW = Win<STENCIL>::n, H = Win<STENCIL>::h;
     const T* __restrict__ src = cons_win ? U : W;
-    constexpr bool AHEAD = kPlainMarch<VAR, RIEMANN, DISS, FLIM>;
+    constexpr bool AHEAD = kPlainMarch<VAR, STENCIL, RIEMANN, DISS, FLIM>;
     constexpr bool CARRY = AHEAD && kCarry<VAR, STENCIL>;
     double win[NW][5], nxt[5], carry[5];
 #pragma unroll
@@ -89,7 +91,38 @@ JFA_WAVES_PER_EU((kPlainMarch<VAR, RIEMANN, DISS, FLIM> ? 2 : 1)) void march_ker
     cr[A] = a0;
     cr[O] = io;
     cr[IN] = iin;
-    if constexpr (DISS) dissipative_face<T, A>(W, G, prm, cr, Fp);
+    // dissipative fluxes: the left cell's temperature and transverse derivatives come from the face below
+    double Tl = 0.0, dl[3][3];
+    auto dissipative = [&](double (&F)[5]) {
+        int64_t bl_, br_;
+        face_cells<A>(G, prm, cr, bl_, br_);
+        double wl[5], wr[5], dr[3][3];
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+            wl[i] = cons_win ? ld(W, i * fs + bl_) : win[H - 1][i];
+            wr[i] = cons_win ? ld(W, i * fs + br_) : win[H][i];
+        }
+        transverse_derivatives<T, A>(W, G, prm, cr, br_, dr);
+        const double Tr = temperature(wr, prm);
+        DissState s;
+        dissipative_state_between<A, true>(G, prm, wl, Tl, dl, wr, Tr, dr, s);
+        dissipative_flux<A, true>(s, G, prm, F);
+        Tl = Tr;
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) dl[i][k] = dr[i][k];
+    };
+    if constexpr (DISS) {
+        int64_t bl_, br_;
+        face_cells<A>(G, prm, cr, bl_, br_);
+        double wl[5];
+#pragma unroll
+        for (int i = 0; i < 5; ++i) wl[i] = cons_win ? ld(W, i * fs + bl_) : win[H - 1][i];
+        Tl = temperature(wl, prm);
+        transverse_derivatives<T, A>(W, G, prm, cr, bl_, dl);
+        dissipative(Fp);
+    }
     // R layout (5, N0, N1, N2)
     const int64_t ncell = (int64_t)G.n[0] * G.n[1] * G.n[2];
     const int64_t rsA = A == 0 ? (int64_t)G.n[1] * G.n[2] : (A == 1 ? (int64_t)G.n[2] : 1);
@@ -124,7 +157,7 @@ JFA_WAVES_PER_EU((kPlainMarch<VAR, RIEMANN, DISS, FLIM> ? 2 : 1)) void march_ker
             cr[A] = a + 1;
             JFA_OPAQUE(cr[O]);  // keeps the neighbours' addresses out of the loop's registers
             JFA_OPAQUE(cr[IN]);
-            dissipative_face<T, A>(W, G, prm, cr, Fn);
+            dissipative(Fn);
         }
 #pragma unroll
         for (int i = 0; i < 5; ++i) {
@@ -249,7 +282,13 @@ __global__ __launch_bounds__(kInnerBlock) void inner_kernel(const T* __restrict_
             cr[IN] = (int)f;
             cr[P] = cP;
             cr[Q] = cQ;
-            dissipative_face<T, IN>(W, G, prm, cr, F);
+            double wl[5], wr[5];
+#pragma unroll
+            for (int i = 0; i < 5; ++i) {
+                wl[i] = cons_win ? ld(W, i * fs + bf - 1) : win[H - 1][i];
+                wr[i] = cons_win ? ld(W, i * fs + bf) : win[H][i];
+            }
+            dissipative_face<T, IN>(W, G, prm, cr, wl, wr, F);
         }
     }
     double Fu[5];
@@ -506,8 +545,10 @@ static int64_t sweeps(const void* W, const void* U, const Geo& G, const Params& 
         // The kernels of the common options hold them as constants; the others (the frozen state and
         // signal speed switches and the face-state limiter cost scalar registers, whose spills cost
         // FINAL 7 % and the x sweep 8 %) keep MARCH + INNER.  1-D grids have no axis to walk along.
-        if (common_scheme<VAR, RIEMANN>(prm) && IN > 0) {
-            const int A = IN == 1 || !G.active[1] ? 0 : 1;
+        const int A = IN == 1 || !G.active[1] ? 0 : 1;
+        // the upper faces of a chunk's rows lie within 32-bit byte offsets of the first one
+        const bool reach = 64 * G.s[A] * (int64_t)sizeof(T) < (int64_t)1 << 32;
+        if (common_scheme<VAR, RIEMANN>(prm) && IN > 0 && reach) {
             FinalPlan plan;
             static int64_t slots = 0;  // the (A, IN) variants hold the same registers and LDS
             if (slots == 0)
