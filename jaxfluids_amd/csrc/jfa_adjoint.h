@@ -1709,7 +1709,7 @@ __global__ __launch_bounds__(kAdjBlock) void adj_march_kernel(const double* __re
 // marching chunk repeats 5 faces of 21), the WENO indicators once per cell (four times a face), and
 // the cell pass needs few registers.  The price is 80 bytes written and read per face, and the cell
 // pass is bound by them (3.6 of the 4.8 TB/s a copy reaches); the face pass is bound by FP64 issue.
-// 128^3, WENO5-Z HLLC, us per stage along x / y / z: 536 / 498 / 338 in one pass, 263 / 250 / 267 in two.
+// 128^3, WENO5-Z HLLC, us per stage along x / y / z: 536 / 498 / 338 in one pass, 250 / 250 / 245 in two.
 template <int VAR, int STENCIL, int RIEMANN>
 constexpr bool kTwoPass = VAR == JFA_PRIMITIVE && (STENCIL == JFA_WENO5_JS || STENCIL == JFA_WENO5_Z) &&
                           RIEMANN != kFluxSplit;

@@ -100,7 +100,7 @@ struct InnerArgs {
 // A wavefront holds 64 consecutive cells of rows along IN and walks along A.  Rows live in LDS, NW - 1
 // of them in a ring (5 fields each): the A window of a lane is its own column of the ring, the IN
 // window of the row that is finished is the row beside the lane's cell, so every cell is loaded from
-// memory once (plus H rows per chunk).  How rows are cut (lane_map):
+// memory once (plus H rows per chunk).  How rows are cut:
 //   packed = 0: each wave takes 64 cells of one row; five cells beside them are loaded as well, and
 //     the flux above its last cell is evaluated for all rows of the chunk before the walk (lane k: row
 //     a0 + k).  No lane idles where the row length is a multiple of 64.
@@ -110,8 +110,8 @@ struct InnerArgs {
 // Loads run ahead: the finish's (scratch RHS, U, U_n) at the top of the row, two faces before their
 // use; the next row's during the A face, once the reconstruction is done with the window.
 //
-// Bound: FP64 issue at the clock the card holds under it (70 % of the cycles issue; 1.97 GHz), about
-// 240 VGPRs (two waves per SIMD; three spill), 2.5 GB read and 1.6 GB written per stage at 256^3.
+// Bound: FP64 issue of two waves per SIMD (250 VGPRs; three spill) at the clock the card holds under it
+// (58 % of the cycles issue; 1.97 GHz), 3.1 GB read and 1.6 GB written per stage at 256^3.
 // Measured there (FP64, sustained, us per stage with the x sweep): CHAR-PRIMITIVE WENO5-Z HLLC 2000
 // with MARCH + INNER, 1460 with this kernel (windows through the caches instead of LDS 1680, the
 // finish's loads after the IN face 1490); PRIMITIVE WENO5-JS 1770 and 1425.  256 x 256: 22.8 and
