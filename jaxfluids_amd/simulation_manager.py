@@ -62,7 +62,10 @@ class SimulationManager:
         self._bufs = None
         self._graph = None
         self._graph_key = None
+        # a step's dt on the host (do_integration_step): pinned, and the event that says it has arrived
         self._dt_host = None
+        if torch.cuda.is_available():
+            self._dt_host = (torch.empty(1, dtype=torch.float64, pin_memory=True), torch.cuda.Event())
         self.wall_clock_times = []
 
     # ------------------------------------------------------------------ buffers
@@ -179,24 +182,17 @@ class SimulationManager:
         if not isinstance(dt, torch.Tensor):
             dt = torch.full((1,), float(dt), dtype=torch.float64, device=W.device)
         # the step overwrites dt: its value goes to the host ahead of the step's kernels, and the wait for
-        # it follows their launch (the GPU would idle for a round trip of 12 us otherwise).  The first step
-        # has nothing to run ahead of and makes the pinned buffer behind its own kernels.
-        ahead = self._dt_host
-        if ahead is None:
-            dt_used = float(dt.item())
-        else:
-            ahead[0].copy_(dt.reshape(1), non_blocking=True)
-            ahead[1].record()
+        # it follows their launch (the GPU would idle for a round trip of 12 us otherwise)
+        dt_host, copied = self._dt_host
+        dt_host.copy_(dt.reshape(1), non_blocking=True)
+        copied.record()
         if self.use_graph and self.fused:
             # the replayed step reads and writes dt in place
             self._capture(W, U, dt).replay()
         else:
             W, U = self._step_kernels(W, U, dt)
-        if ahead is None:
-            self._dt_host = (torch.empty(1, dtype=torch.float64, pin_memory=True), torch.cuda.Event())
-        else:
-            ahead[1].synchronize()
-            dt_used = float(ahead[0])
+        copied.synchronize()
+        dt_used = float(dt_host)
         tcv = tcv._replace(physical_simulation_time=tcv.physical_simulation_time + dt_used,
                            simulation_step=tcv.simulation_step + 1, physical_timestep_size=dt)
         return JaxFluidsBuffers(MaterialFieldBuffers(U, W, mf.temperature), tcv)
