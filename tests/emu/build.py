@@ -14,7 +14,8 @@ SOURCES = [os.path.join(CSRC, f) for f in ("jfa_batch_f64.hip", "jfa_batch_f32.h
                                             "jfa_fused_cons.hip", "jfa_fused_charprim.hip", "jfa_fused_charcons.hip",
                                             "jfa_fused_fsplit.hip")]
 DEPS = SOURCES + [os.path.join(CSRC, f) for f in ("jfa_batch.h", "jfa_common.h", "jfa_device.h", "jfa_adjoint.h",
-                                                  "jfa_dissipative.h", "jfa_fused.h")] + [
+                                                  "jfa_dissipative.h", "jfa_fused.h", "jfa_walk.h")] + [
+    os.path.join(ROOT, "include", "jaxfluids_amd.h"),
     os.path.join(HERE, "emu_runtime.cpp"), os.path.join(HERE, "hip", "hip_runtime.h"), __file__]
 
 
