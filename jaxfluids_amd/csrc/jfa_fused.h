@@ -544,11 +544,12 @@ static int64_t sweeps(const void* W, const void* U, const Geo& G, const Params& 
     if constexpr (kFinal<VAR, STENCIL, RIEMANN, DISS, FLIM>) {
         // The kernels of the common options hold them as constants; the others (the frozen state and
         // signal speed switches and the face-state limiter cost scalar registers, whose spills cost
-        // FINAL 7 % and the x sweep 8 %) keep MARCH + INNER.  1-D grids have no axis to walk along.
+        // FINAL 7 % and the x sweep 8 %) keep MARCH + INNER.  1-D grids have no axis to walk along,
+        // whichever axis is theirs: A is inactive, without halos, and INNER alone evaluates IN.
         const int A = IN == 1 || !G.active[1] ? 0 : 1;
         // the upper faces of a chunk's rows lie within 32-bit byte offsets of the first one
         const bool reach = 64 * G.s[A] * (int64_t)sizeof(T) < (int64_t)1 << 32;
-        if (common_scheme<VAR, RIEMANN>(prm) && IN > 0 && reach) {
+        if (common_scheme<VAR, RIEMANN>(prm) && A < IN && G.active[A] && reach) {
             FinalPlan plan;
             static int64_t slots = 0;  // the (A, IN) variants hold the same registers and LDS
             if (slots == 0)

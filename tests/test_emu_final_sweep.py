@@ -14,7 +14,7 @@ import pytest
 
 from oracle import jxf_oracle as o
 from test_emu_fused import FACES, check_step, emu, fused_step  # noqa: F401 - emu: fixture
-from test_gpu_parity import random_state
+from test_gpu_parity import random_state, rel
 
 SCHEMES = {
     "z-charprim-hllc": dict(stencil="WENO5-Z", variable="CHAR-PRIMITIVE", riemann="HLLC"),
@@ -37,6 +37,50 @@ def test_step(emu, scheme, cells, bcs):  # noqa: F811
     s = o.Setup(gamma=1.4, signal_speed="EINFELDT", frozen_state="ARITHMETIC", bcs=BCS[bcs], **SCHEMES[scheme])
     dom, W0 = random_state(cells, 3, seed=sum(cells), jump=False)
     check_step(emu, dom, s, W0)
+
+
+ONE_DIMENSIONAL = [n for N in (17, 64, 100) for n in ((1, N, 1), (1, 1, N))]
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("cells", ONE_DIMENSIONAL, ids=["x".join(map(str, g)) for g in ONE_DIMENSIONAL])
+@pytest.mark.parametrize("variable", ["PRIMITIVE", "CHAR-PRIMITIVE"])
+@pytest.mark.parametrize("riemann, bcs", [("HLLC", "periodic"), ("RUSANOV", "mixed")])
+def test_one_dimensional(emu, riemann, bcs, variable, cells, dtype):  # noqa: F811
+    """A domain along y or z alone has no second axis to walk along: the step and the right-hand side
+    against the oracle, every access inside the registered buffers.  FP32 storage: a step's state is
+    rounded to float three times, the right-hand side of the rounded state once."""
+    from jaxfluids_amd import _native
+
+    s = o.Setup(gamma=1.4, signal_speed="EINFELDT", frozen_state="ARITHMETIC", stencil="WENO5-Z", variable=variable,
+                riemann=riemann, bcs=BCS[bcs])
+    dom, W0 = random_state(cells, 3, seed=sum(cells), jump=False)
+    if dtype == np.float64:
+        check_step(emu, dom, s, W0)
+    W, U = o.create_buffers(W0, dom, s)
+    dt = o.compute_dt(W, dom, s)
+    Wr, _ = o.rk3_step(W, U, dt, dom, s)
+    Wg, _, _ = fused_step(emu, dom, s, W, U, dt, dtype=dtype)
+    I = dom.interior
+    assert rel(Wg[I].astype(np.float64), Wr[I]) < (1e-12 if dtype == np.float64 else 1e-6)
+
+    emu.jfa_compute_rhs.restype, emu.jfa_compute_rhs.argtypes = _native.SIGNATURES["jfa_compute_rhs"]
+    emu.jfa_rhs_workspace_bytes.restype, emu.jfa_rhs_workspace_bytes.argtypes = _native.SIGNATURES["jfa_rhs_workspace_bytes"]
+    code = _native.F64 if dtype == np.float64 else _native.F32
+    grid = _native.make_grid(dom.cells, dom.nh, dom.dx)
+    scheme = _native.make_scheme(s.variable, s.stencil, s.riemann, s.signal_speed, s.frozen_state, code, s.gamma,
+                                 s.eps_stencil)
+    Wd, Ud = np.ascontiguousarray(W.astype(dtype)), np.ascontiguousarray(U.astype(dtype))
+    rhs = np.full((5,) + dom.cells, np.nan, dtype=dtype)
+    ws = np.zeros(emu.jfa_rhs_workspace_bytes(grid, code), dtype=np.uint8)
+    emu.emu_clear_ranges()
+    for a in (Wd, Ud, rhs, ws):
+        emu.emu_add_range(a.ctypes.data, a.nbytes)
+    assert emu.jfa_compute_rhs(Wd.ctypes.data, Ud.ctypes.data, grid, scheme, 0.0, rhs.ctypes.data, ws.ctypes.data,
+                               ws.nbytes, None) == 0
+    assert emu.emu_violations() == 0, hex(emu.emu_first_violation())
+    want = o.compute_rhs(Wd.astype(np.float64), Ud.astype(np.float64), dom, s, 0.0)
+    assert rel(rhs.astype(np.float64), want) < (1e-12 if dtype == np.float64 else 1e-6)
 
 
 def test_common_options_match_the_general_kernels(emu):  # noqa: F811

@@ -362,6 +362,26 @@ def test_rk3_step_parity_2d(case, bc):
     assert abs(host(dtd)[0] - o.compute_dt(Wr, dom, s)) < 1e-14 * dt
 
 
+@pytest.mark.parametrize("cells", [(1, 17, 1), (1, 1, 17), (1, 130, 1), (1, 1, 130)], ids=lambda c: "x".join(map(str, c)))
+@pytest.mark.parametrize("case", [FLUX_CASES[0], FLUX_CASES[2]], ids="-".join)
+@pytest.mark.parametrize("fused", [True, False])
+def test_rk3_step_parity_1d(case, cells, fused):
+    """1-D domains along y and z: no second axis to walk along, whatever the scheme."""
+    from jaxfluids_amd import SimulationManager
+
+    say(f"[rk3 step 1d] {cells} fused={fused} {case}")
+    dom, W0 = random_state(cells, 3, seed=sum(cells), jump=False)
+    s = _setup(case, {f: ("ZEROGRADIENT" if o.FACE_AXIS[f] in dom.active else "PERIODIC") for f in FACES})
+    s.frozen_state = "ARITHMETIC"
+    sim = SimulationManager(_input_manager(dom, s), fused=fused)
+    W, U = o.create_buffers(W0, dom, s)
+    dt = o.compute_dt(W, dom, s)
+    Wr, Ur = o.rk3_step(W, U, dt, dom, s)
+    Wd, Ud = sim.do_runge_kutta_stages(dev(W), dev(U), torch.full((1,), dt, dtype=torch.float64, device="cuda"))
+    I = dom.interior
+    assert rel(host(Wd)[I], Wr[I]) < TOL and rel(host(Ud)[I], Ur[I]) < TOL
+
+
 def test_fp32_storage_error_stated():
     """FP32 storage (FP64 arithmetic) against the FP64 oracle on one TGV step: the error is
     the float32 rounding of the state, stated here as < 1e-6 relative L-inf."""
