@@ -40,12 +40,26 @@ __device__ __forceinline__ double coef(double c) {
 // and an index computation per neighbour, 109 with this and the neighbours as offsets).  Error against
 // extended precision on the GPU, 4e5 values each of x in [e^-300, e^300] and p of -0.7 .. 3: below
 // 0.57 ulp, mean 0.25 (pow: 1.33 and up to 0.35).
+// Outside 0 < x < infinity as pow; SIGNED: x may be negative, which has a power only for a whole p (NaN
+// otherwise, so a cell of negative temperature shows in the time step).  The faces' temperatures are
+// clamped to positive ones: their power leaves that branch out (it costs 0.5 .. 2.7 % of a viscous stage).
 constexpr double kLn2Hi = 0x1.62e42fefa0000p-1, kLn2Lo = 0x1.cf79abc9e3b3ap-40;
-template <bool SCALAR>
+
+// x^p (p != 0) for x <= 0, an infinite x and NaN, where v = |x|^p if x is finite and not 0
+__device__ __forceinline__ double power_special(double x, double p, double v) {
+    const double h = 0.5 * p, a = fabs(x);
+    const bool whole = rint(p) == p, odd = whole && rint(h) != h;
+    double r = v;
+    if (!(a > 0.0 && a < __builtin_inf())) r = p > 0.0 ? a : __builtin_amdgcn_rcp(a);  // 0, infinity, NaN
+    else if (!whole) r = __builtin_nan("");
+    return odd ? copysign(r, x) : r;
+}
+
+template <bool SCALAR, bool SIGNED>
 __device__ __forceinline__ double power(double x, double p) {
 #pragma clang fp contract(off)
     int k;
-    double m = frexp(x, &k);
+    double m = frexp(SIGNED ? fabs(x) : x, &k);
     const bool low = m < 0.70710678118654757;
     m = low ? m + m : m;
     k = low ? k - 1 : k;
@@ -96,27 +110,32 @@ __device__ __forceinline__ double power(double x, double p) {
     const double c = fma(b * q, E + E, fma(q, ql, ql) + be);
     const double v = ldexp(w + ((u - (w - 1.0)) + ((b - (u - q)) + c)), (int)n2);
     const bool finite = x > 0.0 && x < __builtin_inf();
-    return finite ? v : (p > 0.0 ? x : __builtin_amdgcn_rcp(x));  // 0, infinity, NaN
+    if constexpr (SIGNED) {
+        if (!finite) return power_special(x, p, v);
+        return v;
+    } else {
+        return finite ? v : (p > 0.0 ? x : __builtin_amdgcn_rcp(x));  // 0, infinity, NaN
+    }
 }
 
-template <bool SCALAR = false>
+template <bool SCALAR = false, bool SIGNED = false>
 __device__ __forceinline__ double law_value(double T, const Law& l) {
     if (l.kind == JFA_LAW_SUTHERLAND) {  // material.py:94-96, power3_2 (math/power_functions.py:29-30)
         const double x = T * l.inv_T_ref;
         return l.ref * ((l.T_ref + l.param) / (T + l.param)) * (x * sqrt(x));
     }
-    return l.param == 0.0 ? l.ref : l.ref * power<SCALAR>(T * l.inv_T_ref, l.param);
+    return l.param == 0.0 ? l.ref : l.ref * power<SCALAR, SIGNED>(T * l.inv_T_ref, l.param);
 }
 
-template <bool SCALAR = false>
+template <bool SCALAR = false, bool SIGNED = false>
 __device__ __forceinline__ double viscosity(double T, const Params& prm) {
-    return law_value<SCALAR>(T, prm.mu);
+    return law_value<SCALAR, SIGNED>(T, prm.mu);
 }
 
 // thermal conductivity at temperature T, where mu = viscosity(T)
-template <bool SCALAR = false>
+template <bool SCALAR = false, bool SIGNED = false>
 __device__ __forceinline__ double conductivity(double T, double mu, const Params& prm) {
-    return prm.kappa.kind == JFA_LAW_PRANDTL ? prm.kappa_fac * mu : law_value<SCALAR>(T, prm.kappa);
+    return prm.kappa.kind == JFA_LAW_PRANDTL ? prm.kappa_fac * mu : law_value<SCALAR, SIGNED>(T, prm.kappa);
 }
 
 // Offsets from a cell at coordinate c along axis i to its neighbours above and below: on periodic
@@ -264,9 +283,9 @@ __device__ __forceinline__ void dissipative_face(const T* __restrict__ W, const 
 // cell diffusivities for the time-step limits: nu = mu/rho, alpha = kappa/(rho cp)
 __device__ __forceinline__ void diffusivities(const double w[5], const Params& prm, double& nu, double& alpha) {
     const double T = w[4] / (w[0] * prm.R);
-    const double mu = viscosity<true>(T, prm);
+    const double mu = viscosity<true, true>(T, prm);
     nu = (prm.dissip & 1) ? mu / w[0] : 0.0;
-    alpha = (prm.dissip & 2) ? conductivity<true>(T, mu, prm) / w[0] * prm.inv_cp : 0.0;
+    alpha = (prm.dissip & 2) ? conductivity<true, true>(T, mu, prm) / w[0] * prm.inv_cp : 0.0;
 }
 
 }  // namespace jfa
