@@ -185,6 +185,8 @@ __device__ __forceinline__ void rk3_coeffs(int stage, double& c0, double& c1, do
 // (positive or negative) order like their bit patterns read as unsigned 64-bit integers, so a
 // 64-bit atomicMax on the bits is an exact, order-independent max that keeps a NaN.
 __device__ __forceinline__ double nan_max(double a, double b) { return (a > b || a != a) ? a : b; }
+// The smallest of the time step's limits, NaN if one of them is, as the reference's minimum.
+__device__ __forceinline__ double nan_min(double a, double b) { return (a < b || a != a) ? a : b; }
 
 __device__ __forceinline__ double wave_sum(const double w[5], const int act[3], double gamma) {
     const double c = sound_speed(w[4], w[0], gamma);

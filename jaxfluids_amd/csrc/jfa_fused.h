@@ -408,8 +408,8 @@ __global__ __launch_bounds__(1024) void dt_from_parts_kernel(const double* __res
             for (int i = 1; i < (int)(blockDim.x >> 6); ++i) mx[q] = nan_max(mx[q], sm[q][i]);
         }
         double d = dx_min / (mx[0] + eps);
-        if (dissip & 1) d = fmin(d, 3.0 / 14.0 * dx_min * dx_min / (mx[1] + eps));
-        if (dissip & 2) d = fmin(d, 0.1 * dx_min * dx_min / (mx[2] + eps));
+        if (dissip & 1) d = nan_min(d, 3.0 / 14.0 * dx_min * dx_min / (mx[1] + eps));
+        if (dissip & 2) d = nan_min(d, 0.1 * dx_min * dx_min / (mx[2] + eps));
         dt[0] = d * cfl;
     }
 }

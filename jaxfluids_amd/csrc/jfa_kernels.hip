@@ -314,8 +314,8 @@ __global__ void zero_slot_kernel(unsigned long long* slot) {
 __global__ void dt_finalize_kernel(const unsigned long long* slot, double dx_min, double cfl, double eps, int dissip,
                                    double* dt) {
     double d = dx_min / (__longlong_as_double((long long)slot[0]) + eps);
-    if (dissip & 1) d = fmin(d, 3.0 / 14.0 * dx_min * dx_min / (__longlong_as_double((long long)slot[1]) + eps));
-    if (dissip & 2) d = fmin(d, 0.1 * dx_min * dx_min / (__longlong_as_double((long long)slot[2]) + eps));
+    if (dissip & 1) d = nan_min(d, 3.0 / 14.0 * dx_min * dx_min / (__longlong_as_double((long long)slot[1]) + eps));
+    if (dissip & 2) d = nan_min(d, 0.1 * dx_min * dx_min / (__longlong_as_double((long long)slot[2]) + eps));
     dt[0] = d * cfl;
 }
 

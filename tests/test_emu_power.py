@@ -80,6 +80,9 @@ LAWS = {
     "power": o.Transport(R=1.0, mu_ref=2e-2, T_ref=1.0, mu_exp=0.76, bulk_viscosity=1e-2, prandtl=0.71),
     "power-heat-law": o.Transport(R=1.0, mu_ref=2e-2, T_ref=1.0, mu_exp=-0.7, kappa_ref=1e-2, kappa_exp=0.5),
     "sutherland": o.Transport(R=1.0, mu_ref=2e-2, T_ref=1.0, mu_sutherland=0.4, prandtl=0.71),
+    # a diffusivity that is a number at any temperature: the wave speed alone is NaN
+    "constant": o.Transport(R=1.0, mu_ref=2e-2, T_ref=1.0, mu_exp=0.0, prandtl=0.71),
+    "square": o.Transport(R=1.0, mu_ref=2e-2, T_ref=1.0, mu_exp=2.0, prandtl=0.71),
 }
 
 
