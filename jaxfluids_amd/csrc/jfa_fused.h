@@ -282,11 +282,13 @@ __global__ __launch_bounds__(kInnerBlock) void inner_kernel(const T* __restrict_
             cr[IN] = (int)f;
             cr[P] = cP;
             cr[Q] = cQ;
+            int64_t bl, br;  // windows of U say nothing about W's halos: its cells as the faces wrap them
+            face_cells<IN>(G, prm, cr, bl, br);
             double wl[5], wr[5];
 #pragma unroll
             for (int i = 0; i < 5; ++i) {
-                wl[i] = cons_win ? ld(W, i * fs + bf - 1) : win[H - 1][i];
-                wr[i] = cons_win ? ld(W, i * fs + bf) : win[H][i];
+                wl[i] = cons_win ? ld(W, i * fs + bl) : win[H - 1][i];
+                wr[i] = cons_win ? ld(W, i * fs + br) : win[H][i];
             }
             dissipative_face<T, IN>(W, G, prm, cr, wl, wr, F);
         }
