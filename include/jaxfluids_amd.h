@@ -251,7 +251,7 @@ int jfa_rk3_stage(void* U, const void* U_n, const void* rhs, void* W, const jfa_
                   void* stream);
 
 /* jfa_rk3_stage of U into U_out, and prim(U_out) into W_out; the halos of U_out and W_out are copies of
- * those of U and W.  The outputs must not overlap the inputs. */
+ * those of U and W.  Outputs that overlap an input or one another are refused (JFA_EINVAL). */
 int jfa_rk3_stage_into(const void* W, const void* U, const void* U_n, const void* rhs, void* W_out, void* U_out,
                        const jfa_grid* grid, const jfa_scheme* scheme, int32_t stage, const double* dt_dev,
                        double dt_host, void* stream);

@@ -6,6 +6,7 @@
 // all arithmetic is FP64.
 #include <hip/hip_runtime.h>
 
+#include <cstdint>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -531,6 +532,12 @@ int jfa_rk3_stage(void* U, const void* U_n, const void* rhs, void* W, const jfa_
     return check_launch();
 }
 
+// whether two memory ranges share a byte
+static bool overlap(const void* a, size_t na, const void* b, size_t nb) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return x < y + nb && y < x + na;
+}
+
 int jfa_rk3_stage_into(const void* W, const void* U, const void* U_n, const void* rhs, void* W_out, void* U_out,
                        const jfa_grid* grid, const jfa_scheme* scheme, int32_t stage, const double* dt_dev,
                        double dt_host, void* stream) {
@@ -540,7 +547,13 @@ int jfa_rk3_stage_into(const void* W, const void* U, const void* U_n, const void
     rc = check_scheme(scheme);
     if (rc) return rc;
     if (!W || !U || !rhs || !W_out || !U_out || stage < 0 || stage > 2 || (stage > 0 && !U_n)) return JFA_EINVAL;
-    if (W_out == W || U_out == U) return JFA_EINVAL;
+    const size_t item = scheme->dtype == JFA_F32 ? sizeof(float) : sizeof(double), state = (size_t)(5 * G.fs) * item;
+    const size_t nrhs = (size_t)5 * G.n[0] * G.n[1] * G.n[2] * item;
+    for (const void* out : {W_out, U_out})
+        if (overlap(out, state, W, state) || overlap(out, state, U, state) || overlap(out, state, rhs, nrhs) ||
+            (stage > 0 && overlap(out, state, U_n, state)))
+            return JFA_EINVAL;
+    if (overlap(W_out, state, U_out, state)) return JFA_EINVAL;
     const dim3 g = flat_grid(G.fs);
     hipStream_t st = (hipStream_t)stream;
     if (scheme->dtype == JFA_F32)

@@ -74,6 +74,12 @@ class RungeKutta3(TimeIntegrator):
         theirs, so neither buffer is copied beforehand.
         """
         U_in = integration_buffers.euler_buffers.conservatives
+        if primitives is not None:
+            for name, t in (("primitives", primitives), ("primitives_out", primitives_out)):
+                if t is not None and (t.dtype != U_in.dtype or t.device != U_in.device or t.shape != U_in.shape or
+                                      not t.is_contiguous() or not U_in.is_contiguous()):
+                    raise ValueError(f"{name} must be laid out as the conservatives: contiguous, of their dtype, "
+                                     "device and shape")
         U = U_in.clone() if primitives is None else torch.empty_like(U_in)
         Un = initial_stage_buffers.euler_buffers.conservatives if stage > 0 else None
         rhs = rhs_buffers.euler_buffers.conservatives.contiguous()
