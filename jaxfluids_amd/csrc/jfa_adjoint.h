@@ -127,13 +127,22 @@ __device__ __forceinline__ void weno5_cell_vjp(double a, double b, double c, dou
         tau = fabs(b0 - b2);
     }
     const double p12 = q1 * q2, p02 = q0 * q2, p01 = q0 * q1;
-    const double P = p01 * q2;
-    const double rP = rcp(P);
     double e0 = p12, e1 = p02, e2 = p01;
-    if constexpr (STENCIL == JFA_WENO5_Z) {
+    double i0, i1, i2;  // 1 / q_k; WENO-JS without the product of all three, which the forward stencil does not form
+    if constexpr (STENCIL == JFA_WENO5_Z) {  // (it holds differences to the sixth power, WENO-JS's to the twelfth)
+        const double P = p01 * q2;
+        const double rP = rcp(P);
         e0 = fma(tau, p12, P);
         e1 = fma(tau, p02, P);
         e2 = fma(tau, p01, P);
+        i0 = p12 * rP;
+        i1 = p02 * rP;
+        i2 = p01 * rP;
+    } else {
+        const double r01 = rcp(p01);
+        i0 = q1 * r01;
+        i1 = q0 * r01;
+        i2 = rcp(q2);
     }
     // hi = c + N_h / M_h, lo = c + N_l / M_l (weno5_state)
     const double gh0 = fma(5.0 / 6.0, d1, (-1.0 / 3.0) * d0), gh1 = fma(2.0, d2, d1), gh2 = fma(-0.5, d3, 2.0 * d2);
@@ -145,7 +154,7 @@ __device__ __forceinline__ void weno5_cell_vjp(double a, double b, double c, dou
     const double eb1 = fma(nh, gh1 - 6.0 * xh, nl * (gl1 - 6.0 * xl));
     const double eb2 = fma(nh, gh2 - 3.0 * xh, nl * (gl0 - xl));
     const double T0 = eb0 * p12, T1 = eb1 * p02, T2 = eb2 * p01;
-    const double t0 = T0 * (p12 * rP), t1 = T1 * (p02 * rP), t2 = T2 * (p01 * rP);  // T_k / q_k
+    const double t0 = T0 * i0, t1 = T1 * i1, t2 = T2 * i2;  // T_k / q_k
     double g0, g1, g2;  // cotangents of 4 beta_k
     if constexpr (STENCIL == JFA_WENO5_JS) {
         g0 = -2.0 * b0 * t0;

@@ -59,3 +59,26 @@ def test_written_equals_added_to_zero(emu, cells, nh, bcs, variable):  # noqa: F
     for a, w in zip(added, written):
         assert np.array_equal(a[dom.interior], w[dom.interior])
     assert fn(*args, 4, ws.ctypes.data, ws.nbytes, None) == _native.JFA_EINVAL
+
+
+@pytest.mark.parametrize("stencil", ["WENO5-JS", "WENO5-Z"])
+def test_range(emu, stencil):  # noqa: F811
+    """A flow's gradient in other units: speeds times 2^45 (pressures of 1e27) give the same cotangents, scaled
+    by powers of two, to the roundings of the reciprocals.  On a uniform state the weights are the linear ones at
+    any epsilon that the forward stencils take (its square is a normal number)."""
+    dom = o.Domain((9, 8, 1), ((0.0, 1.0), (0.0, 1.1), (0.0, 0.9)), nh=3)
+    lam = np.zeros((5,) + dom.shape)
+    lam[dom.interior] = np.random.default_rng(7).standard_normal((5,) + dom.cells)
+
+    def gradient(W0, eps, a):
+        units = np.array([1.0, a, a, a, a * a]).reshape(5, 1, 1, 1)
+        s = o.Setup(gamma=1.4, stencil=stencil, variable="PRIMITIVE", riemann="HLLC", signal_speed="EINFELDT",
+                    bcs=dict(zip(FACES, PERIODIC)), eps_stencil=eps)
+        W = np.ascontiguousarray(o.create_buffers(W0 * units, dom, s)[0])
+        return run_vjp(emu, dom, s, W, lam / units, 1, 1e-3 / a)[0][dom.interior] * units
+
+    smooth = smooth_state(dom, 3)
+    uniform = np.ones((5,) + dom.cells) * np.array([1.0, 0.3, -0.2, 0.0, 1.5]).reshape(5, 1, 1, 1)
+    for W0, eps, a in ((smooth, 1e-30, 2.0 ** 45), (uniform, 1e-140 if stencil == "WENO5-JS" else 1e-90, 1.0)):
+        got, want = gradient(W0, eps, a), gradient(W0, 1e-30, 1.0)
+        assert np.max(np.abs(got - want)) <= 1e-12 * np.max(np.abs(want)), (eps, a)
