@@ -34,6 +34,54 @@ from .space_solver import SpaceSolver
 from .time_integration import compute_time_step_size
 
 
+class _DtToHost:
+    """The dt of a step on its way to the host: pinned copies and the events that say they have arrived.
+
+    A step takes a free copy and gives it back, so steps of several threads, or one inside another, keep
+    their own; there are as many as steps were ever under way at once.  They are kept per device, the
+    events being a device's.  The first step on a device reads dt directly and the copy is made behind its
+    kernels, unless the program had the GPU in use when the manager was built: building one does not
+    initialise the GPU (a program may still choose its device, or fork).  Copies of a manager make
+    their own."""
+
+    def __init__(self) -> None:
+        self._free = {}  # device -> [(pinned copy, event)]
+        if torch.cuda.is_initialized():
+            self._add(torch.device("cuda", torch.cuda.current_device()))
+
+    def __reduce__(self):
+        return (_DtToHost, ())
+
+    def _add(self, device) -> None:
+        arrived = torch.cuda.Event()
+        arrived.record(torch.cuda.current_stream(device))  # creates the event
+        with torch.inference_mode(False):  # later steps may run outside of it
+            copy = torch.empty(1, dtype=torch.float64, device="cpu", pin_memory=True)
+        self._free.setdefault(device, []).append((copy, arrived))
+
+    def send(self, dt: torch.Tensor):
+        """Starts the copy of dt, behind the work of the current stream."""
+        try:
+            copy, arrived = self._free[dt.device].pop()
+        except (KeyError, IndexError):
+            return float(dt.item())
+        copy.copy_(dt.reshape(1), non_blocking=True)
+        arrived.record(torch.cuda.current_stream(dt.device))
+        return copy, arrived
+
+    def receive(self, sent, device) -> float:
+        """The value of dt that `send` was given."""
+        if isinstance(sent, float):
+            if not self._free.get(device):
+                self._add(device)
+            return sent
+        copy, arrived = sent
+        arrived.synchronize()
+        value = float(copy)
+        self._free[device].append(sent)
+        return value
+
+
 class SimulationManager:
     def __init__(self, input_manager, fused: bool = True, use_graph: bool = False) -> None:
         im = input_manager
@@ -62,10 +110,7 @@ class SimulationManager:
         self._bufs = None
         self._graph = None
         self._graph_key = None
-        # a step's dt on the host (do_integration_step): pinned, and the event that says it has arrived
-        self._dt_host = None
-        if torch.cuda.is_available():
-            self._dt_host = (torch.empty(1, dtype=torch.float64, pin_memory=True), torch.cuda.Event())
+        self._dt_to_host = _DtToHost()
         self.wall_clock_times = []
 
     # ------------------------------------------------------------------ buffers
@@ -183,16 +228,13 @@ class SimulationManager:
             dt = torch.full((1,), float(dt), dtype=torch.float64, device=W.device)
         # the step overwrites dt: its value goes to the host ahead of the step's kernels, and the wait for
         # it follows their launch (the GPU would idle for a round trip of 12 us otherwise)
-        dt_host, copied = self._dt_host
-        dt_host.copy_(dt.reshape(1), non_blocking=True)
-        copied.record()
+        sent = self._dt_to_host.send(dt)
         if self.use_graph and self.fused:
             # the replayed step reads and writes dt in place
             self._capture(W, U, dt).replay()
         else:
             W, U = self._step_kernels(W, U, dt)
-        copied.synchronize()
-        dt_used = float(dt_host)
+        dt_used = self._dt_to_host.receive(sent, dt.device)
         tcv = tcv._replace(physical_simulation_time=tcv.physical_simulation_time + dt_used,
                            simulation_step=tcv.simulation_step + 1, physical_timestep_size=dt)
         return JaxFluidsBuffers(MaterialFieldBuffers(U, W, mf.temperature), tcv)
