@@ -1162,10 +1162,15 @@ __device__ __forceinline__ void face_state_vjp_at(const double* __restrict__ W, 
                                                   const double mu[5], const Params& prm, double gl[5], double gr[5],
                                                   double fz[FZ_N]) {
     double win[6][5], wl[5], wr[5];
+    // Field by field: in the lane-parallel sweeps across the rows a load touches 64 cache lines, which the
+    // field's other five loads share; the lines of all five fields at once exceed the L1 (CONSERVATIVE
+    // WENO5-Z HLLC, us per sweep across the rows of 512 x 500: 163 with the cells in the outer loop, 143 so).
 #pragma unroll
-    for (int k = 0; k < 6; ++k)
+    for (int i = 0; i < 5; ++i) {
 #pragma unroll
-        for (int i = 0; i < 5; ++i) win[k][i] = ld(W, i * fs + br + (int64_t)(k - 3) * sa);
+        for (int k = 0; k < 6; ++k) win[k][i] = ld(W, i * fs + br + (int64_t)(k - 3) * sa);
+        JFA_SCHED_BARRIER();
+    }
 #pragma unroll
     for (int i = 0; i < 5; ++i) {  // the face's two cells (read by the CHAR-CONSERVATIVE frozen state)
         wl[i] = win[2][i];
