@@ -1723,7 +1723,7 @@ __global__ __launch_bounds__(kAdjBlock) void adj_march_kernel(const double* __re
 // marching chunk repeats 5 faces of 21), the WENO indicators once per cell (four times a face), and
 // the cell pass needs few registers.  The price is 80 bytes written and read per face, and the cell
 // pass is bound by them (3.6 of the 4.8 TB/s a copy reaches); the face pass is bound by FP64 issue.
-// 128^3, WENO5-Z HLLC, us per stage along x / y / z: 536 / 498 / 338 in one pass, 250 / 250 / 245 in two.
+// 128^3, WENO5-Z HLLC, us per stage along x / y / z: 536 / 498 / 338 in one pass, 240 / 239 / 235 in two.
 template <int VAR, int STENCIL, int RIEMANN>
 constexpr bool kTwoPass = VAR == JFA_PRIMITIVE && (STENCIL == JFA_WENO5_JS || STENCIL == JFA_WENO5_Z) &&
                           RIEMANN != kFluxSplit;
@@ -2040,7 +2040,7 @@ __device__ __forceinline__ void dissipative_state_of_cell(const double* __restri
 // dissipative cotangent, added to gW, and the sum X[3 i + k](c) of the transverse-derivative
 // cotangents Gt of its faces (interior layout, ncell per field), gathered by adj_update_kernel.
 // What the six faces share (c's state, temperature and transverse derivatives) is formed once: bound by
-// loads through L1, 160 a cell against 324 with each face on its own (128^3, us: 265 and 302).
+// loads through L1, 160 a cell against 324 with each face on its own (128^3, us: 257 and 302).
 template <int UNUSED = 0>
 __global__ __launch_bounds__(kBlock) JFA_WAVES_PER_EU(3) void adj_dissip_cell_kernel(const double* __restrict__ W,
                                                                  const double* __restrict__ lam, Geo G, Params prm,

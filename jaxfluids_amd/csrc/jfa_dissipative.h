@@ -25,7 +25,7 @@ namespace jfa {
 // each into vector registers before its fma, or keeps them all in scalar registers around a loop and
 // spills others for it: a viscous sweep takes 223 VGPRs so and 177 with SCALAR.  Where many faces stand
 // in one block the asm keeps them from being interleaved: the reverse's cell kernel spills with SCALAR
-// (128^3, us: 331 against 250).
+// (128^3, us: 331 against 257).
 template <bool SCALAR>
 __device__ __forceinline__ double coef(double c) {
     if constexpr (!SCALAR) return c;

@@ -40,9 +40,12 @@ constexpr int kMarchBlock = 256;
 // ahead, before the step's stores, so no wait covers a store (256^3 CHAR-PRIMITIVE WENO5-Z HLLC, us
 // per sweep along x / y: 507 / 589 loading at the top of the step, 433 / 476 ahead, 397 / - with the
 // common options as constants).  The plain convective variants are held to two waves per SIMD so that
-// nothing spills; the common ones fit three by themselves.  So are the dissipative ones with a WENO5
-// stencil and HLLC or Rusanov (128^3 viscous PRIMITIVE, us per sweep: 97 loading at the top of the
-// step without carried states, 89 with both); the others need more registers and do neither.
+// nothing spills; the common ones fit three by themselves.  For the others, held to three waves and
+// loading at the top of the step before, us per stage at 128^3: CHAR-PRIMITIVE with the ROE frozen state
+// 274 then, 240 so; PRIMITIVE HLL 316, 222; TENO5 330, 320; WENO7-JS 579, 558; CONSERVATIVE 233, 216.  So
+// are the dissipative ones with a WENO5 stencil and HLLC or Rusanov (128^3 viscous PRIMITIVE, us per
+// sweep: 97 loading at the top of the step without carried states, 85 with both); the rest need more
+// registers and do neither.
 template <int VAR, int STENCIL, int RIEMANN, bool DISS, bool FLIM>
 constexpr bool kPlainMarch = !(FLIM || VAR == JFA_CHAR_CONSERVATIVE || RIEMANN == kFluxSplit) &&
                              (!DISS || ((STENCIL == JFA_WENO5_JS || STENCIL == JFA_WENO5_Z) &&
